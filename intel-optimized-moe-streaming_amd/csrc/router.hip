@@ -10,11 +10,13 @@
 //            multiplies by fl32(w), moe_layer.py:70,85-86); a non-finite or
 //            non-positive exponential sum gives 1/k each (router.py:161-166).
 //
-// Two launches.  k_route_scores: each workgroup owns 4/SPLIT experts and a
+// Two launches.  k_route_scores (up to a hundred or so tokens): each workgroup owns 4/SPLIT experts and a
 // group of tokens; SPLIT waves share one expert row, each summing a contiguous
 // share of the hidden dimension with 16-byte loads (a lane's chain, then a
 // fixed DPP tree over the wave), and the shares are added in wave order, so
-// the summation order of a score is fixed for a given SPLIT.
+// the summation order of a score is fixed for a given SPLIT.  k_route_scores_mfma
+// (more tokens): the same FP32 products and sums as a matrix product on the FP32
+// matrix instructions, also in a fixed order.
 // k_route_select: one wavefront per token takes the top k by k rounds of a
 // wave maximum over (score, expert) keys (route_topk.h): NaN ranks above every
 // number, as np.argsort places NaN last (a NaN among the selected then makes
@@ -113,6 +115,131 @@ __global__ __launch_bounds__(64 * RS_WAVES) void k_route_scores(const float* __r
     }
 }
 
+// Scores of many tokens on v_mfma_f32_32x32x2_f32 (FP32 in, FP32 sums).  A
+// workgroup owns 32 TB tokens x 32 experts; its sixteen waves share the hidden
+// dimension, each a contiguous slice of a multiple of 32 columns, and read their
+// operands straight into registers: the instruction takes row l % 32 of both
+// operands at column l / 32, so with the columns of a group of eight dealt as
+// 0..3 to the low and 4..7 to the high half of the wave (the same for both
+// operands) a lane's 16-byte load feeds four instructions.  No LDS staging and
+// no barrier before the waves' partial tiles are added.
+//
+// Summation order: chains of CH columns, joined as a tree over each 32 (TB = 1) or
+// added in turn, then the sixteen waves' sums as a tree.  The vector kernel's
+// chains are H / 64 columns under six tree levels.  CH = 16 from H = 1536 on and
+// 8 from 512 on is no less accurate (relative error against 64 bits at 512 tokens
+// x 256 experts, vector and matrix kernel: 1.23e-7 and 1.04e-7 at H = 2048,
+// 1.00e-7 and 0.90e-7 at 1024, 0.86e-7 both at 512); below 512 the vector
+// kernel's chains are shorter still (0.78e-7 and 0.81e-7 at 256) and it stays.
+// Bound by the FP32 matrix rate (2 T E H operations, 14 us for 2048 x 256 scores
+// of 2048 columns) and, below some 256 tiles, by one workgroup's own chain (17 us
+// there).  That size: 133 -> 34 us; 512 x 256 x 2048: 37.6 -> 17.2 us.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int RM_WAVES = 16;
+constexpr int RM_STEP = 32;   // columns of a pass
+
+// Columns C0 .. C0 + N - 1 of a pass (in the order the lanes hold them): chains
+// of CH, joined as a tree.  MFMA c of group s takes columns 8 s + c and 8 s + 4 + c.
+template <int C0, int N, int CH>
+__device__ __forceinline__ f32x16 rm_tree(const float4 (&av)[RM_STEP / 8], const float4 (&bv)[RM_STEP / 8]) {
+    if constexpr (N > CH) {
+        const f32x16 l = rm_tree<C0, N / 2, CH>(av, bv);
+        return l + rm_tree<C0 + N / 2, N / 2, CH>(av, bv);
+    } else {
+        f32x16 p;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) p[i] = 0.0f;
+#pragma unroll
+        for (int c = C0; c < C0 + N; c += 2)
+            p = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float*)&av[c / 8])[c % 8 / 2],
+                                                     ((const float*)&bv[c / 8])[c % 8 / 2], p, 0, 0, 0);
+        return p;
+    }
+}
+
+template <int TB, int CH>
+__global__ __launch_bounds__(64 * RM_WAVES) void k_route_scores_mfma(const float* __restrict__ x, int n_tokens,
+                                                                     int hidden, const float* __restrict__ w,
+                                                                     int n_experts, float* __restrict__ scores,
+                                                                     int per, int n_etiles) {
+    __shared__ float part[RM_WAVES][TB][32][32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, l32 = lane & 31;
+    // workgroup i runs on XCD i % 8: the expert tiles of one token tile have
+    // indices that agree mod 8, so its rows are read into one XCD's L2
+    const int j = blockIdx.x / 8;
+    const int et = j % n_etiles, tt = (j / n_etiles) * 8 + blockIdx.x % 8;
+    const int t0 = tt * 32 * TB, e0 = et * 32;
+    if (t0 >= n_tokens) return;
+    // rows past the last repeat it and are not stored
+    const float* wr = w + (int64_t)min(e0 + l32, n_experts - 1) * hidden + 4 * half;
+    const float* xr[TB];
+#pragma unroll
+    for (int b = 0; b < TB; ++b) xr[b] = x + (int64_t)min(t0 + 32 * b + l32, n_tokens - 1) * hidden + 4 * half;
+
+    f32x16 acc[TB];
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[b][i] = 0.0f;
+    const int k1 = min(hidden, (wave + 1) * per);
+    for (int k = wave * per; k < k1; k += RM_STEP) {
+        float4 bv[RM_STEP / 8], av[TB][RM_STEP / 8];
+#pragma unroll
+        for (int s = 0; s < RM_STEP / 8; ++s) {
+            // columns past the last enter as zeros (of both operands)
+            const bool in = k + 8 * s + 4 * half < k1;
+            const int o = in ? k + 8 * s : 0;
+            const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float4 bw = *(const float4*)(wr + (in ? o : -4 * half));
+            bv[s] = in ? bw : z;
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                const float4 ax = *(const float4*)(xr[b] + (in ? o : -4 * half));
+                av[b][s] = in ? ax : z;
+            }
+        }
+        if constexpr (TB == 1) {
+            acc[0] += rm_tree<0, RM_STEP, CH>(av[0], bv);
+        } else {   // the token blocks' chains in turn (the tree's registers would spill)
+#pragma unroll
+            for (int c0 = 0; c0 < RM_STEP; c0 += CH) {
+                f32x16 p[TB];
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) p[b][i] = 0.0f;
+#pragma unroll
+                for (int c = c0; c < c0 + CH; c += 2)
+#pragma unroll
+                    for (int b = 0; b < TB; ++b)
+                        p[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float*)&av[b][c / 8])[c % 8 / 2],
+                                                                    ((const float*)&bv[c / 8])[c % 8 / 2], p[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < TB; ++b) acc[b] += p[b];
+            }
+        }
+    }
+    // D layout: register 4 g + i of lane l holds row 8 g + 4 (l / 32) + i, column l % 32
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) part[wave][b][8 * (i / 4) + 4 * half + i % 4][l32] = acc[b][i];
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < TB; ++b) {
+        const int row = threadIdx.x >> 5, col = threadIdx.x & 31;
+        const int t = t0 + 32 * b + row, e = e0 + col;
+        float v[RM_WAVES];
+#pragma unroll
+        for (int i = 0; i < RM_WAVES; ++i) v[i] = part[i][b][row][col];
+#pragma unroll
+        for (int d = 1; d < RM_WAVES; d *= 2)
+#pragma unroll
+            for (int i = 0; i < RM_WAVES; i += 2 * d) v[i] += v[i + d];
+        if (t < n_tokens && e < n_experts) scores[(int64_t)t * n_experts + e] = v[0];
+    }
+}
+
 template <int NM>
 __global__ __launch_bounds__(64 * SEL_WAVES) void k_route_select(const float* __restrict__ scores, int n_tokens,
                                                                  int n_experts, int top_k, int32_t* __restrict__ ids,
@@ -142,6 +269,20 @@ static void launch_scores(const float* x, int n_tokens, int hidden, const float*
                        n_experts, scores);
 }
 
+template <int TB>
+static void launch_scores_mfma(const float* x, int n_tokens, int hidden, const float* w, int n_experts, float* scores,
+                               hipStream_t stream) {
+    const int n_etiles = (n_experts + 31) / 32, n_ttiles = (n_tokens + 32 * TB - 1) / (32 * TB);
+    const int per = ((hidden + RM_WAVES - 1) / RM_WAVES + RM_STEP - 1) / RM_STEP * RM_STEP;
+    const dim3 grid((unsigned)((n_ttiles + 7) / 8 * 8 * n_etiles)), block(64 * RM_WAVES);
+    if (hidden >= 1536)
+        hipLaunchKernelGGL((k_route_scores_mfma<TB, 16>), grid, block, 0, stream, x, n_tokens, hidden, w, n_experts,
+                           scores, per, n_etiles);
+    else
+        hipLaunchKernelGGL((k_route_scores_mfma<TB, 8>), grid, block, 0, stream, x, n_tokens, hidden, w, n_experts,
+                           scores, per, n_etiles);
+}
+
 template <int NM>
 static void launch_select(const float* scores, int n_tokens, int n_experts, int top_k, int32_t* ids, float* weights,
                           hipStream_t stream) {
@@ -150,16 +291,31 @@ static void launch_select(const float* scores, int n_tokens, int n_experts, int 
 }
 
 // Few tokens: four waves per expert row, so the n_experts x 4 waves spread
-// over the chip, and as many token accumulators as there are tokens (up to 8);
-// many tokens: one wave per expert over 16 tokens, so each row is read once
-// per 16 tokens.
+// over the chip, and as many token accumulators as there are tokens (up to 8).
+// Above 32 tokens the number of scores decides, each step's work being
+// proportional to the hidden size on all sides (us at hidden 2048):
+//   up to 8192      the same, eight tokens at a time (64 x 16: 3.3, one wave per
+//                   expert over 16 tokens 7.2; 33 x 256: 5.7 and 7.7; 64 x 256: 7.9 and 7.7)
+//   below 49152     one wave per expert over 16 tokens, so each row is read
+//                   once per 16 tokens (128 x 256: 11.4, matrix kernel 16.8)
+//   from 49152 on   the matrix kernel (200 x 256: 16.9, vector 19.6; at hidden
+//                   1024 11.8 and 11.2, 512 x 256 12.1 and 19.8); 64 tokens a
+//                   workgroup where 32 would give well over one workgroup a CU
+//                   (2048 x 256 at hidden 1024: 20.8, 32 tokens 26.9; 1024 x
+//                   256: 17.2 and 14.7)
+constexpr int64_t RS_FEW_SCORES = 8192, RM_MIN_SCORES = 49152;
+constexpr int64_t RM_WIDE_TILES = 384;
 hipError_t launch_route_scores(const float* x, int n_tokens, int hidden, const float* w, int n_experts, float* scores,
                                hipStream_t stream) {
+    const int64_t n = (int64_t)n_tokens * n_experts;
     if (n_tokens == 1) launch_scores<4, 1>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else if (n_tokens == 2) launch_scores<4, 2>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else if (n_tokens <= 4) launch_scores<4, 4>(x, n_tokens, hidden, w, n_experts, scores, stream);
-    else if (n_tokens <= 32) launch_scores<4, 8>(x, n_tokens, hidden, w, n_experts, scores, stream);
-    else launch_scores<1, 16>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else if (n_tokens <= 32 || n <= RS_FEW_SCORES) launch_scores<4, 8>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else if (n < RM_MIN_SCORES || hidden < 512) launch_scores<1, 16>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else if (hidden >= 1024 && (int64_t)((n_tokens + 31) / 32) * ((n_experts + 31) / 32) > RM_WIDE_TILES)
+        launch_scores_mfma<2>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else launch_scores_mfma<1>(x, n_tokens, hidden, w, n_experts, scores, stream);
     return hipGetLastError();
 }
 

@@ -248,3 +248,26 @@ def test_routed_decode_matches_the_oracle_layer(oracle_mod, E, types, sh_types, 
         ref = oracle_layer(oracle_mod, layer, host, shared, X[t], o_ids, o_w)
         err = np.abs(y[t] - ref).max() / max(np.abs(ref).max(), 1e-30)
         assert err <= 1e-3, f"token {t}: {err}"
+
+
+@pytest.mark.parametrize("T,H,E,k", [
+    (192, 512, 256, 8),     # the first size on the matrix kernel: whole tiles, half the waves idle
+    (1025, 516, 49, 4),     # one token and 17 experts past a tile, four columns past a pass
+    (257, 1540, 193, 6),    # the longer chains, every edge ragged
+    (2048, 1024, 256, 8),   # 64 tokens a workgroup, chains of 8
+    (1633, 2044, 250, 8),   # 64 tokens a workgroup, chains of 16, every edge ragged
+])
+def test_route_scores_many_tokens(T, H, E, k):
+    """Scores against float64: an FP32 sum of H products in any order is off by at
+    most H eps sum|x w| (eps = 2^-24), and each edge has inputs of its own size, so
+    a column, row or expert taken twice or left out shows."""
+    rng = np.random.default_rng(T + H + E)
+    x = rng.standard_normal((T, H)).astype(np.float32)
+    w = (rng.standard_normal((H, E)) * 0.05).astype(np.float32)
+    x[-1] *= 3.0
+    x[:, -1] += 2.0
+    w[:, -1] += 0.5
+    _, _, scores = gpu_route(x, w, k, with_scores=True)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    bound = H * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
+    assert np.all(np.abs(scores - x64 @ w64) <= bound)
