@@ -15,10 +15,6 @@ constexpr int64_t WS_HEAD_BYTES = (int64_t)N_FLAGS * 4;
 
 constexpr int ROUTE_PROLOGUE_MAX_EXPERTS = 256;   // 4 router scores per lane
 
-constexpr int ROWS_A = 8;    // intermediate rows per workgroup, kernel A
-constexpr int ROWS_W = 4;    // hidden rows per wavefront, kernel B
-constexpr int ROWS_B = 4 * ROWS_W;
-
 struct DecodeParams {
     // The first 64 bytes are what the fast kernels need before their first
     // loads (the token, the expert ids, the activations and the geometry of

@@ -661,3 +661,48 @@ def test_intermediate_2048_over_slot_limit_falls_back(hip, oracle_mod):
     for tok in range(2):
         want = oracle_layer(oracle_mod, layer, host, shared, X[tok], ids[tok].tolist(), ws[tok].tolist())
         assert oracle_mod.max_relative_error(got[tok], want) <= TOL, tok
+
+
+@pytest.mark.parametrize("gt,ut,dt,H,I,sh_I,k,T", [
+    (12, 12, 14, 1536, 768, 768, 6, 1),     # 64 and 32 lanes a row, three units a lane
+    (8, 8, 8, 96, 32, 64, 3, 2),            # rows shorter than the lanes, one block of inter
+    (11, 13, 8, 768, 1280, 1280, 2, 3),     # gate and up of different types, two passes in B
+    (13, 13, 13, 1792, 2304, 256, 2, 1),    # seven units a lane in two passes, nine in three
+    (14, 14, 12, 5120, 256, 512, 9, 1),     # ten units in three passes, more slots than waves, the
+                                            # shared expert's rows on other lanes than the routed ones
+    (20, 20, 8, 352, 160, 160, 1, 2),       # IQ4_NL, lanes with and without a second unit
+])
+def test_generic_sizes(hip, oracle_mod, gt, ut, dt, H, I, sh_I, k, T):
+    """The FP32 kernels over sizes that are no power of two, against float64.
+
+    A row's sum is two chains of at most 40 products a lane under six tree
+    levels: about sqrt(20 + 7) 2^-24 = 3e-7 of its terms' norm, which two sums
+    in turn and Q4_K's offsets (terms a few times the result) take to ~2e-6."""
+    t = {"gate": gt, "up": ut, "down": dt}
+    E = 10
+    # (scales at which the FP16 graph stays finite)
+    layer, host, shared = make_layer(H + I + k, E, H, I, t, shared_types=t, sh_I=sh_I, scale=0.0005)
+    rng = np.random.default_rng(H + 3 * I + k)
+    X = rng.standard_normal((T, H)).astype(np.float32)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)])
+    ws = rng.dirichlet(np.ones(k), size=T).astype(np.float32)
+    print(f"generic sizes {t} H={H} I={I} shared {sh_I} k={k} T={T}", flush=True)
+    old = hip.mqh_set_decode_path(1)
+    try:
+        got, st = run(layer, X, ids, ws)
+        assert st == 0
+        half, st = run(layer, X, ids, ws, fp16=1) if 20 not in (gt, ut, dt) else (None, 0)
+        assert st == 0
+    finally:
+        hip.mqh_set_decode_path(old)
+    sh_t = {r: shared[r] for r in ROLES}
+    for tok in range(T):
+        gate = 1.0 / (1.0 + np.exp(-float(X[tok].astype(np.float64) @ shared["gate_inp"])))
+        want = gate * _f64_expert(oracle_mod, sh_t, t, X[tok], H, sh_I)
+        for e, w in zip(ids[tok], ws[tok]):
+            want = want + float(w) * _f64_expert(oracle_mod, host_expert(host, layer, int(e)), t, X[tok], H, I)
+        err = np.linalg.norm(got[tok] - want) / np.linalg.norm(want)
+        assert err <= 4e-6, (tok, err)
+        if half is not None:
+            want16 = oracle_layer(oracle_mod, layer, host, shared, X[tok], ids[tok].tolist(), ws[tok].tolist(), fp16=1)
+            assert oracle_mod.max_relative_error(half[tok], want16) <= TOL, tok
