@@ -585,7 +585,11 @@ int64_t mqh_moe_prefill_workspace_bytes(int n_tokens, int top_k, int n_experts, 
     if (n_tokens <= 0 || top_k < 0 || top_k > 64 || n_experts <= 0 || hidden <= 0 || intermediate <= 0 ||
         (has_shared != 0 && has_shared != 1) || (top_k == 0 && !has_shared))
         return ST_ARG;
-    return prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared).total;
+    // (the types are not known here: room for either tile width)
+    int64_t need = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, false).total;
+    if (prefill_wide_size(n_tokens, top_k, n_experts, hidden, intermediate, has_shared))
+        need = std::max(need, prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, true).total);
+    return need;
 }
 
 int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up, int down_type, const void* down,
@@ -618,7 +622,9 @@ int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up
     p.has_shared = has_shared;
     p.sh_gate_type = sh_gate_type; p.sh_up_type = sh_up_type; p.sh_down_type = sh_down_type;
     if (!prefill_supported(p)) return ST_TYPE;
-    const PrefillLayout L = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared);
+    const bool wide = prefill_wide_types(down_type, has_shared, sh_down_type) &&
+                      prefill_wide_size(n_tokens, top_k, n_experts, hidden, intermediate, has_shared);
+    const PrefillLayout L = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, wide);
     if (workspace_bytes < L.total) return ST_WORKSPACE;
 
     uint8_t* WS = (uint8_t*)workspace;
@@ -633,7 +639,9 @@ int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up
     p.act = (float*)(WS + L.act_off); p.ypair = (float*)(WS + L.ypair_off);
     p.xhi = (uint16_t*)(WS + L.xhi_off); p.xlo = (uint16_t*)(WS + L.xlo_off);
     p.xsum = (uint32_t*)(WS + L.xsum_off); p.xexp = (int*)(WS + L.xexp_off);
-    p.max_tiles = L.max_tiles;
+    p.ahi = (uint16_t*)(WS + L.ahi_off); p.alo = (uint16_t*)(WS + L.alo_off);
+    p.asum = (uint32_t*)(WS + L.asum_off); p.aexp = (int*)(WS + L.aexp_off);
+    p.max_tiles = L.max_tiles; p.tile = L.tile;
     const KernelEvents ev = t_events;
     t_events = KernelEvents();
     return launch_prefill(p, (hipStream_t)stream, ev) == hipSuccess ? ST_OK : ST_HIP;

@@ -86,6 +86,7 @@ inline WorkspaceLayout decode_workspace_layout(int n_tokens, int top_k, int inte
 #endif
 constexpr int PREFILL_TILE = MQH_PREFILL_TILE;
 static_assert(PREFILL_TILE == 8 || PREFILL_TILE == 16, "prefill tiles of 8 or 16 tokens");
+constexpr int PREFILL_WIDE = 64;   // tile width of the kernels for many tokens per expert
 constexpr int PREFILL_MAX_EXPERTS = 1024;
 
 struct PrefillParams {
@@ -114,8 +115,8 @@ struct PrefillParams {
     float* sh_scale;        // [n_tokens]
     int* tiles;             // [max_tiles x 4]: expert, first pair, token count, 0
     int* n_tiles;           // [1]
-    int* tile_tok;          // [max_tiles x PREFILL_TILE]: token of column c of tile i (stale past the tile's count)
-    int* tile_dst;          // [max_tiles x PREFILL_TILE]: its output row t S + s (token t, slot s)
+    int* tile_tok;          // [max_tiles x tile]: token of column c of tile i (stale past the tile's count)
+    int* tile_dst;          // [max_tiles x tile]: its output row t S + s (token t, slot s)
     float* act;             // [P x inter] SwiGLU activations, in sorted pair order
     float* ypair;           // [P x hidden] expert outputs, row t S + s
     // the tokens as the gate/up kernel's B operand, made once per token by the
@@ -127,15 +128,25 @@ struct PrefillParams {
     uint32_t* xsum;
     int* xexp;
     int max_tiles;
+    int tile;               // tile width: PREFILL_TILE or PREFILL_WIDE
+    // wide tiles: the activations as the down kernel's B operand (rows in
+    // sorted pair order), as the token planes are
+    uint16_t* ahi;
+    uint16_t* alo;
+    uint32_t* asum;
+    int* aexp;
 };
 
 struct PrefillLayout {
     int64_t flags_off, scale_off, tiles_off, ntiles_off, tok_off, dst_off, act_off, ypair_off;
-    int64_t xhi_off, xlo_off, xsum_off, xexp_off, total;
-    int max_tiles;
+    int64_t xhi_off, xlo_off, xsum_off, xexp_off, ahi_off, alo_off, asum_off, aexp_off, total;
+    int max_tiles, tile;
 };
 
-PrefillLayout prefill_layout(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared);
+// Whether a prompt's size, and a layer's types, are the wide tiles'
+bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared);
+bool prefill_wide_types(int down_type, int has_shared, int sh_down_type);
+PrefillLayout prefill_layout(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, bool wide);
 bool prefill_supported(const PrefillParams& p);
 
 // Optional HIP events recorded at the start and end of the two GEMM kernels of

@@ -16,6 +16,8 @@
 //                          SwiGLU fused.
 //   P2 k_prefill_down      (H/128) x max_tiles workgroups: 128 output rows x one tile.
 //   P3 k_prefill_combine   grid (H/256, T): the weighted sum in top-k order.
+// With many tokens per expert the tiles are 64 tokens and P1/P2 are the kernels
+// of moe_prefill_wide.hip.
 //
 // P1/P2 are MFMA GEMMs (v_mfma_f32_16x16x32_f16, FP32 accumulate) whose weight
 // operand is built in registers straight from the quantized blocks as exact
@@ -25,14 +27,12 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
-#include <utility>
 
 #include "kquant_frag.h"
 #include "moe_decode.h"
+#include "moe_prefill.h"
 
 namespace mqh {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int PF_WAVES = 8;      // waves per workgroup of the GEMM kernels
 constexpr int PF_ROWS_GU = 64;   // gate/up rows per workgroup: 4 waves on gate, 4 on up
@@ -92,6 +92,17 @@ constexpr int pf_occupancy(int lds_bytes) {
     return (160 * 1024 / lds_bytes) * PF_WAVES / 4 < 8 ? (160 * 1024 / lds_bytes) * PF_WAVES / 4 : 8;
 }
 
+// Tiles of PREFILL_WIDE tokens (moe_prefill_wide.hip) from PF_WIDE_TOKENS
+// (token, slot) pairs per expert on average (the shared expert counts as one),
+// and PF_WIDE_PAIRS in all.  Layer times in us, 64-token and 16-token tiles:
+//   Q4_K/Q6_K, BF16  18 an expert 303/298, 36 366/423, 72 555/715
+//   Q3_K, FP32       18 310/286, 36 399/468, 72 596/791
+//   Q5_K, FP32       16 275/258, 32 326/405, 64 514/689
+//   Q6_K, FP32       18 433/396, 36 538/601, 72 836/1078
+// and with few experts too few workgroups: 256 tokens of 16 experts (2304
+// pairs) 126/120 in Q3_K, 512 of 60 (4608) 205/208.
+constexpr int64_t PF_WIDE_TOKENS = 32, PF_WIDE_PAIRS = 4096;
+
 #ifndef PF_OCC_GU
 #define PF_OCC_GU
 #endif
@@ -99,148 +110,10 @@ constexpr int pf_occupancy(int lds_bytes) {
 #define PF_OCC_DOWN
 #endif
 
-template <int... Ms, class F>
-__device__ __forceinline__ void pf_unroll(std::integer_sequence<int, Ms...>, F&& f) {
-    (f(std::integral_constant<int, Ms>{}), ...);
-}
-
-__device__ __forceinline__ float pf_silu_mul(float g, float u) {
-    const float e = __builtin_amdgcn_exp2f(-g * 1.4426950408889634f);
-    return (g * __builtin_amdgcn_rcpf(1.0f + e)) * u;
-}
-
 __device__ __forceinline__ float pf_sigmoid(float v) {
     if (v >= 0.0f) return 1.0f / (1.0f + expf(-v));
     const float e = expf(v);
     return e / (1.0f + e);
-}
-
-__device__ __forceinline__ float pf_wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
-__device__ __forceinline__ float pf_wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// ------------------------------------------------------------ token staging
-//
-// One wave stages token row `row` of src (K values, FP32 or BF16) as LDS column
-// j of the B operand: high plane xh[j][K + PF_PAD], low plane xl (SPLIT only),
-// and the 32-column sub-block sums / 32 as [block][j][hi 0..7 | lo 0..7] in xs
-// (block-major, so the 16 token columns of one block sit in distinct banks).
-// A lane owns 8 consecutive values per 512-column pass.  The loads
-// (pf_stage_load) and the rest (pf_stage_finish, or pf_stage_planes into
-// device memory) are separate.
-template <int K, bool BF16>
-struct PfStageRaw {
-    static constexpr int NIT = K >= 512 ? K / 512 : 1;
-    uint4 r[NIT][BF16 ? 1 : 2];
-};
-
-// live = false (a token column past the tile's count): every lane reads the
-// row's first values, one request per instruction instead of a row's worth
-template <int K, bool BF16>
-__device__ __forceinline__ void pf_stage_load(const void* src, int64_t row, bool live, PfStageRaw<K, BF16>& raw) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int it = 0; it < PfStageRaw<K, BF16>::NIT; ++it) {
-        // lanes past K (K = 256) read the row's first values again (in bounds, unused)
-        const int c = live ? (512 * it + 8 * lane) % K : 0;
-        if constexpr (BF16) {
-            raw.r[it][0] = *(const uint4*)((const uint16_t*)src + row * K + c);
-        } else {
-            raw.r[it][0] = *(const uint4*)((const float*)src + row * K + c);
-            raw.r[it][1] = *(const uint4*)((const float*)src + row * K + c + 4);
-        }
-    }
-}
-
-// Hands the loaded words through an empty asm statement placed after the
-// weight prefetch: everything computed from them is then ordered after the
-// prefetch (the instruction selector is otherwise free to put the row's
-// arithmetic, and its wait for the row, ahead of the prefetch loads).
-template <int K, bool BF16>
-__device__ __forceinline__ void pf_stage_pin(PfStageRaw<K, BF16>& raw) {
-#pragma unroll
-    for (int it = 0; it < PfStageRaw<K, BF16>::NIT; ++it)
-#pragma unroll
-        for (int j = 0; j < (BF16 ? 1 : 2); ++j)
-            __asm__ volatile("" : "+v"(raw.r[it][j].x), "+v"(raw.r[it][j].y), "+v"(raw.r[it][j].z), "+v"(raw.r[it][j].w));
-}
-
-// The values of pass `it` (8 per lane) from the loaded words; zero past K
-template <int K, bool BF16>
-__device__ __forceinline__ void pf_raw_vals(const PfStageRaw<K, BF16>& raw, int it, int c, float v[8]) {
-    if constexpr (BF16) {
-        const uint32_t w[4] = {raw.r[it][0].x, raw.r[it][0].y, raw.r[it][0].z, raw.r[it][0].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[2 * e] = __uint_as_float(w[e] << 16);
-            v[2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
-        }
-    } else {
-        const uint4 a = raw.r[it][0], b = raw.r[it][1];
-        v[0] = __uint_as_float(a.x); v[1] = __uint_as_float(a.y); v[2] = __uint_as_float(a.z); v[3] = __uint_as_float(a.w);
-        v[4] = __uint_as_float(b.x); v[5] = __uint_as_float(b.y); v[6] = __uint_as_float(b.z); v[7] = __uint_as_float(b.w);
-    }
-    if (c >= K) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-    }
-}
-
-// The row's scale exponent k (its max |value| to [2^13, 2^14), frag_exp); with
-// gvec set, also x_row . gvec (FP32, unscaled) in every lane, else 0.
-template <int K, bool BF16>
-__device__ __forceinline__ int pf_row_exp(const PfStageRaw<K, BF16>& raw, const float* gvec, float& gdot_out) {
-    constexpr int NIT = PfStageRaw<K, BF16>::NIT;
-    const int lane = threadIdx.x & 63;
-    float amax = 0.0f, gdot = 0.0f;
-#pragma unroll
-    for (int it = 0; it < NIT; ++it) {
-        const int c = 512 * it + 8 * lane;
-        float v[8];
-        pf_raw_vals(raw, it, c, v);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
-        if (gvec != nullptr && c < K) {
-            const float4 g0 = *(const float4*)(gvec + c), g1 = *(const float4*)(gvec + c + 4);
-            gdot = fmaf(v[0], g0.x, gdot); gdot = fmaf(v[1], g0.y, gdot);
-            gdot = fmaf(v[2], g0.z, gdot); gdot = fmaf(v[3], g0.w, gdot);
-            gdot = fmaf(v[4], g1.x, gdot); gdot = fmaf(v[5], g1.y, gdot);
-            gdot = fmaf(v[6], g1.z, gdot); gdot = fmaf(v[7], g1.w, gdot);
-        }
-    }
-    gdot_out = pf_wave_sum(gdot);
-    return frag_exp(pf_wave_max(amax));
-}
-
-// Pass `it` of the row at scale 2^-k: the lane's 8 values as FP16 high and low
-// parts, and the sum of its 32-column sub-block (the same in lanes 4m .. 4m+3)
-// as an FP16 (high, low) pair.
-template <int K, bool BF16>
-__device__ __forceinline__ void pf_split_pass(const PfStageRaw<K, BF16>& raw, int it, int k, h8_t& hi, h8_t& lo,
-                                              _Float16& sh, _Float16& sl) {
-    const int c = 512 * it + 8 * (threadIdx.x & 63);
-    float v[8];
-    pf_raw_vals(raw, it, c, v);
-    float s = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        _Float16 h, l;
-        frag_split(v[e], k, h, l);
-        hi[e] = h;
-        lo[e] = l;
-        s += ldexpf(v[e], -k);
-    }
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    frag_split(s, 5, sh, sl);
 }
 
 // Stages the row as LDS column j; the arithmetic runs for a dead column too
@@ -269,34 +142,6 @@ __device__ __forceinline__ void pf_stage_finish(const PfStageRaw<K, BF16>& raw, 
         }
     }
     if (live && lane == 0) s_exp[j] = k;
-}
-
-// The same staging of token t into the token planes in device memory (the
-// route pass makes them once per token; every gate/up workgroup of the token's
-// tiles then copies them into LDS with no arithmetic).  Returns x_t . gvec.
-template <int K, bool BF16, bool SPLIT>
-__device__ __forceinline__ float pf_stage_planes(const PfStageRaw<K, BF16>& raw, int64_t t, const PrefillParams& p,
-                                                 const float* gvec) {
-    constexpr int NIT = PfStageRaw<K, BF16>::NIT;
-    const int lane = threadIdx.x & 63;
-    float gdot;
-    const int k = pf_row_exp(raw, gvec, gdot);
-#pragma unroll
-    for (int it = 0; it < NIT; ++it) {
-        const int c = 512 * it + 8 * lane;
-        h8_t hi, lo;
-        _Float16 sh, sl;
-        pf_split_pass(raw, it, k, hi, lo, sh, sl);
-        if (c < K) {
-            *(h8_t*)((_Float16*)p.xhi + t * K + c) = hi;
-            if constexpr (SPLIT) *(h8_t*)((_Float16*)p.xlo + t * K + c) = lo;
-            if ((lane & 3) == 0)
-                p.xsum[t * (K / 32) + (c >> 5)] =
-                    (uint32_t)__builtin_bit_cast(uint16_t, sh) | (uint32_t)__builtin_bit_cast(uint16_t, sl) << 16;
-        }
-    }
-    if (lane == 0) p.xexp[t] = k;
-    return gdot;
 }
 
 // A token column of the gate/up kernel's B operand as the route pass left it:
@@ -609,6 +454,7 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
     __shared__ int toff[PREFILL_MAX_EXPERTS];
     __shared__ int wsum[16][2];
     const int T = p.n_tokens, K = p.top_k, E = p.n_experts, TK = T * K;
+    const int W = p.tile, wl = 31 - __builtin_clz(W);   // tile width
     const int e = threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (blockIdx.x > 0) {
         constexpr int H = NBH * 256;
@@ -617,7 +463,7 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
         PfStageRaw<H, XBF16> r;
         pf_stage_load<H, XBF16>(p.x, t, true, r);
         const float* gv = p.has_shared ? p.sh_gate_inp : nullptr;
-        const float gd = pf_stage_planes<H, XBF16, !XBF16>(r, t, p, gv);
+        const float gd = pf_stage_planes<H, XBF16, !XBF16>(r, t, PfPlanePtrs{p.xhi, p.xlo, p.xsum, p.xexp}, gv);
         if (p.has_shared && lane == 0) p.sh_scale[t] = gv != nullptr ? pf_sigmoid(gd) : 1.0f;
         return;
     }
@@ -639,7 +485,7 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
     }
     __syncthreads();
     // exclusive scans of pair counts and tile counts over experts
-    const int c = e < E ? cnt[e] : 0, tc = (c + PREFILL_TILE - 1) / PREFILL_TILE;
+    const int c = e < E ? cnt[e] : 0, tc = (c + W - 1) >> wl;
     int ic = c, it = tc;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -656,17 +502,17 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
     // the shared expert's tiles come first (tile j: tokens 16 j .. 16 j + 15):
     // they are the fullest tiles and, with a shared expert of another type, the
     // slowest, so they start in the launch's first round rather than its tail
-    const int nsh = p.has_shared ? (T + PREFILL_TILE - 1) / PREFILL_TILE : 0;
+    const int nsh = p.has_shared ? (T + W - 1) >> wl : 0;
     const int first = bc + ic - c, tfirst = nsh + bt + it - tc;
     if (e < E) {
         off[e] = first;
         toff[e] = tfirst;
         for (int j = 0; j < tc; ++j)
             ((int4*)p.tiles)[tfirst + j] =
-                make_int4(e, first + PREFILL_TILE * j, min(PREFILL_TILE, c - PREFILL_TILE * j), 0);
+                make_int4(e, first + W * j, min(W, c - W * j), 0);
     }
     for (int j = threadIdx.x; j < nsh; j += PF_ROUTE_THREADS)
-        ((int4*)p.tiles)[j] = make_int4(-1, TK + PREFILL_TILE * j, min(PREFILL_TILE, T - PREFILL_TILE * j), 0);
+        ((int4*)p.tiles)[j] = make_int4(-1, TK + W * j, min(W, T - W * j), 0);
     if (threadIdx.x == 0) *p.n_tiles = nsh + tott;
     __syncthreads();
     // pair order inside an expert follows the atomics; a pair's result does not
@@ -678,13 +524,13 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
         const int id = j < PF_ROUTE_IDS ? idr[j < PF_ROUTE_IDS ? j : 0] : p.ids[i];
         if (id >= 0 && id < E) {
             const int k = atomicAdd(&fill[id], 1);
-            const int c = (toff[id] + k / PREFILL_TILE) * PREFILL_TILE + k % PREFILL_TILE;
+            const int c = (toff[id] << wl) + k;
             p.tile_tok[c] = i / K;
             p.tile_dst[c] = (i / K) * p.S + i % K;
         }
     }
     if (p.has_shared) {
-        // column c of shared tile j is token PREFILL_TILE j + c
+        // column c of shared tile j is token W j + c
         for (int t = threadIdx.x; t < T; t += PF_ROUTE_THREADS) {
             p.tile_tok[t] = t;
             p.tile_dst[t] = t * p.S + K;
@@ -918,26 +764,43 @@ bool prefill_supported(const PrefillParams& p) {
     return true;
 }
 
-PrefillLayout prefill_layout(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared) {
+bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared) {
+    const int64_t P = (int64_t)n_tokens * (top_k + (has_shared ? 1 : 0));
+    // (the wide kernels' row offsets into the planes are 32 bits)
+    return P >= PF_WIDE_TOKENS * ((top_k > 0 ? n_experts : 0) + (has_shared ? 1 : 0)) && P >= PF_WIDE_PAIRS &&
+           P * std::max(hidden, inter) < ((int64_t)1 << 32);
+}
+
+bool prefill_wide_types(int down_type, int has_shared, int sh_down_type) {
+    return down_type != T_Q8_0 && !(has_shared && sh_down_type == T_Q8_0);
+}
+
+PrefillLayout prefill_layout(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, bool wide) {
     PrefillLayout L;
     const int S = top_k + (has_shared ? 1 : 0);
     const int64_t P = (int64_t)n_tokens * S;
     const int64_t TK = (int64_t)n_tokens * top_k;
-    L.max_tiles = (int)(std::min<int64_t>(n_experts, TK) + (TK + PREFILL_TILE - 1) / PREFILL_TILE +
-                        (has_shared ? (n_tokens + PREFILL_TILE - 1) / PREFILL_TILE : 0));
+    L.tile = wide ? PREFILL_WIDE : PREFILL_TILE;
+    const int64_t W = L.tile;
+    L.max_tiles = (int)(std::min<int64_t>(n_experts, TK) + (TK + W - 1) / W + (has_shared ? (n_tokens + W - 1) / W : 0));
     L.flags_off = 0;
     L.scale_off = align256(WS_HEAD_BYTES);
     L.tiles_off = align256(L.scale_off + (int64_t)n_tokens * 4);
     L.ntiles_off = align256(L.tiles_off + (int64_t)std::max(L.max_tiles, 1) * 16);
     L.tok_off = align256(L.ntiles_off + 4);
-    L.dst_off = align256(L.tok_off + (int64_t)std::max(L.max_tiles, 1) * PREFILL_TILE * 4);
-    L.act_off = align256(L.dst_off + (int64_t)std::max(L.max_tiles, 1) * PREFILL_TILE * 4);
+    L.dst_off = align256(L.tok_off + (int64_t)std::max(L.max_tiles, 1) * W * 4);
+    L.act_off = align256(L.dst_off + (int64_t)std::max(L.max_tiles, 1) * W * 4);
     L.ypair_off = align256(L.act_off + P * inter * 4);
     L.xhi_off = align256(L.ypair_off + P * hidden * 4);
     L.xlo_off = align256(L.xhi_off + (int64_t)n_tokens * hidden * 2);
     L.xsum_off = align256(L.xlo_off + (int64_t)n_tokens * hidden * 2);
     L.xexp_off = align256(L.xsum_off + (int64_t)n_tokens * (hidden / 32) * 4);
-    L.total = align256(L.xexp_off + (int64_t)n_tokens * 4);
+    const int64_t PA = wide ? P : 0;   // rows with activation planes
+    L.ahi_off = align256(L.xexp_off + (int64_t)n_tokens * 4);
+    L.alo_off = align256(L.ahi_off + PA * inter * 2);
+    L.asum_off = align256(L.alo_off + PA * inter * 2);
+    L.aexp_off = align256(L.asum_off + PA * (inter / 32) * 4);
+    L.total = align256(L.aexp_off + PA * 4);
     return L;
 }
 
@@ -1051,6 +914,11 @@ hipError_t launch_prefill(const PrefillParams& p, hipStream_t s, const KernelEve
 #undef MQH_ROUTE
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
+    if (p.tile == PREFILL_WIDE) {
+        if ((err = launch_prefill_wide(p, s, ev)) != hipSuccess) return err;
+        hipLaunchKernelGGL(k_prefill_combine, dim3((p.hidden + 255) / 256, p.n_tokens), dim3(256), 0, s, p);
+        return hipGetLastError();
+    }
     switch (p.gate_type) {
         case T_Q4_K: launch_p1_t<T_Q4_K>(p, s, ev); break;
         case T_Q5_K: launch_p1_t<T_Q5_K>(p, s, ev); break;

@@ -294,3 +294,48 @@ def test_prefill_q8_0_down_without_shared(oracle_mod, hip, shape):
     got, st = run_prefill(layer, X, ids, ws, use_shared=False)
     assert st == 0
     check(oracle_mod, layer, host, None, X, ids, ws, got, f"Q8_0 down {shape}")
+
+
+@pytest.mark.parametrize("types,sh,shape,x_bf16", [
+    ((12, 14), "same", (2048, 512), True),
+    ((12, 8), "none", (512, 256), False),    # (Q8_0 down projections stay on 16-token tiles)
+    ((11, 11), "q6k", (1024, 512), False),
+    ((13, 12), "same", (256, 1024), False),
+    ((14, 13), "same", (512, 512), True),
+    ((11, 14), "q6k", (512, 2048), True),
+    ((13, 14), "none", (256, 256), True),
+])
+def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
+    """Many tokens per expert (64-token tiles): experts of 0, 1, 16, 17, 32, 33,
+    62 and 161 tokens per 161, so every number of column blocks, full and with
+    one column, and one super-block of hidden or intermediate up to eight.  The
+    161 tokens are checked against the oracle; the prompt repeats them until its
+    size is the wide tiles' (every repetition's rows are the same bits: a pair's
+    result does not depend on its column)."""
+    (gt, dt), (H, I) = types, shape
+    kinds = {"gate": gt, "up": gt, "down": dt}
+    st = {"none": None, "same": kinds, "q6k": {"gate": 14, "up": 14, "down": 14}}[sh]
+    layer, host, shared = make_layer(7100 + gt + dt + H, 8, H, I, kinds, shared_types=st)
+    rng = np.random.default_rng(gt * dt + H)
+    first = np.repeat([1, 2, 3, 4, 5, 6], [1, 16, 17, 32, 33, 62])
+    T = len(first)
+    first = rng.permutation(first)
+    # the repetitions' second pairs go to expert 0 and theirs, too, to 7: the
+    # other experts keep the counts above
+    reps = 4096 // (T * 2) + 1
+    X1 = rng.standard_normal((T, H)).astype(np.float32) * rng.uniform(0.01, 30, (T, 1)).astype(np.float32)
+    X = np.concatenate([X1] * reps)
+    ids = np.zeros((T * reps, 2), np.int64)
+    ids[:T, 1] = first
+    ids[T:, 1] = 7
+    ws = rng.dirichlet(np.ones(2), size=T * reps).astype(np.float32)
+    ws[2 * T:] = np.tile(ws[T:2 * T], (reps - 2, 1))
+    if x_bf16:
+        X = bf16(X)
+    print(f"prefill wide tiles types={types} shared={sh} H={H} I={I} T={len(X)} bf16={x_bf16}", flush=True)
+    got, status = run_prefill(layer, X, ids, ws, x_bf16=x_bf16)
+    assert status == 0
+    check(oracle_mod, layer, host, shared, X[:T], ids[:T], ws[:T], got[:T], f"wide {types} {shape}")
+    check(oracle_mod, layer, host, shared, X[T:T + 9], ids[T:T + 9], ws[T:T + 9], got[T:T + 9], "expert 7")
+    for r in range(2, reps):
+        np.testing.assert_array_equal(got[r * T:(r + 1) * T], got[T:2 * T])
