@@ -439,7 +439,11 @@ static int pf_grid(int nch, int max_tiles) { return nch * ((max_tiles + PF_XCDS 
 // ------------------------------------------------------------ P0
 
 constexpr int PF_ROUTE_THREADS = 1024;   // one workgroup (a constant: blockDim.x costs a memory round trip)
-constexpr int PF_ROUTE_IDS = 4;          // (token, slot) ids a routing thread keeps in registers
+// Ids a routing thread loads at a time, all in flight together (one at a time,
+// the route pass of a 4096-token prompt's 32768 ids took 50 us, a memory round
+// trip per 1024; 43 us so, the rest its scattered stores); the first batch stays
+// in registers for the second pass.
+constexpr int PF_ROUTE_IDS = 8;
 
 // Tokens a staging workgroup takes: one wave each on waves 0..3 (one a SIMD;
 // sixteen a workgroup measured 1.2 us longer for the route pass at 128 tokens)
@@ -469,19 +473,31 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
     }
     if (e < E) { cnt[e] = 0; fill[e] = 0; }
     __syncthreads();
-    // a thread's first PF_ROUTE_IDS ids stay in registers for the second pass
-    // (one memory round trip fewer on the pass's path); the rest are re-read
     int idr[PF_ROUTE_IDS];
+    // f(i, id) for the thread's pairs i of the batch from i0, first loading their
+    // ids (unless `have`)
+    const auto batch = [&](int i0, bool have, int (&id)[PF_ROUTE_IDS], auto&& f) {
+        if (!have)
 #pragma unroll
-    for (int j = 0; j < PF_ROUTE_IDS; ++j) {
-        const int i = threadIdx.x + j * PF_ROUTE_THREADS;
-        idr[j] = i < TK ? p.ids[i] : 0;
-    }
-    for (int i = threadIdx.x; i < TK; i += PF_ROUTE_THREADS) {
-        const int j = (i - threadIdx.x) / PF_ROUTE_THREADS;
-        const int id = j < PF_ROUTE_IDS ? idr[j < PF_ROUTE_IDS ? j : 0] : p.ids[i];
+            for (int j = 0; j < PF_ROUTE_IDS; ++j) {
+                const int i = i0 + j * PF_ROUTE_THREADS;
+                id[j] = i < TK ? p.ids[i] : 0;
+            }
+#pragma unroll
+        for (int j = 0; j < PF_ROUTE_IDS; ++j) {
+            const int i = i0 + j * PF_ROUTE_THREADS;
+            if (i < TK) f(i, id[j]);
+        }
+    };
+    const auto count = [&](int, int id) {
         if (id < 0 || id >= E) atomicOr(&p.flags[FLAG_BAD_ID], 1);
         else atomicAdd(&cnt[id], 1);
+    };
+    constexpr int BATCH = PF_ROUTE_IDS * PF_ROUTE_THREADS;
+    batch(threadIdx.x, false, idr, count);
+    for (int i0 = threadIdx.x + BATCH; i0 < TK; i0 += BATCH) {
+        int id[PF_ROUTE_IDS];
+        batch(i0, false, id, count);
     }
     __syncthreads();
     // exclusive scans of pair counts and tile counts over experts
@@ -519,15 +535,18 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
     // depend on its column in the tile, so outputs do not depend on it.  Each
     // column also gets the output row of its (token, slot), where the down
     // kernel writes it and the combine reads it.
-    for (int i = threadIdx.x; i < TK; i += PF_ROUTE_THREADS) {
-        const int j = (i - threadIdx.x) / PF_ROUTE_THREADS;
-        const int id = j < PF_ROUTE_IDS ? idr[j < PF_ROUTE_IDS ? j : 0] : p.ids[i];
+    const auto place = [&](int i, int id) {
         if (id >= 0 && id < E) {
             const int k = atomicAdd(&fill[id], 1);
             const int c = (toff[id] << wl) + k;
             p.tile_tok[c] = i / K;
             p.tile_dst[c] = (i / K) * p.S + i % K;
         }
+    };
+    batch(threadIdx.x, true, idr, place);
+    for (int i0 = threadIdx.x + BATCH; i0 < TK; i0 += BATCH) {
+        int id[PF_ROUTE_IDS];
+        batch(i0, false, id, place);
     }
     if (p.has_shared) {
         // column c of shared tile j is token W j + c
