@@ -440,10 +440,10 @@ static int pf_grid(int nch, int max_tiles) { return nch * ((max_tiles + PF_XCDS 
 
 constexpr int PF_ROUTE_THREADS = 1024;   // one workgroup (a constant: blockDim.x costs a memory round trip)
 // Ids a routing thread loads at a time, all in flight together (one at a time,
-// the route pass of a 4096-token prompt's 32768 ids took 50 us, a memory round
-// trip per 1024; 43 us so, the rest its scattered stores); the first batch stays
-// in registers for the second pass.
-constexpr int PF_ROUTE_IDS = 8;
+// the route pass of a 4096-token prompt's 32768 ids took 50 us; 46 us so, the
+// rest its scattered stores); the first batch stays in registers for the second
+// pass.
+constexpr int PF_ROUTE_IDS = 4;
 
 // Tokens a staging workgroup takes: one wave each on waves 0..3 (one a SIMD;
 // sixteen a workgroup measured 1.2 us longer for the route pass at 128 tokens)
