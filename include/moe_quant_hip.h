@@ -182,6 +182,12 @@ int mqh_moe_decode_routed(int gate_type, const void* gate, int up_type, const vo
                           float* weights, float* y, int fp16_graph, void* workspace,
                           int64_t workspace_bytes, void* stream);
 
+/* mqh_moe_decode and mqh_moe_decode_routed with their arguments, in order, as
+ * 64-bit words (27 and 29; pointers as integers, absent ones 0): one argument
+ * to marshal for a foreign-function caller. */
+int mqh_moe_decode_words(const int64_t* args);
+int mqh_moe_decode_routed_words(const int64_t* args);
+
 /* Router kernels of the calling thread's last mqh_moe_decode_routed: 1 (the
  * select step ran inside the gate/up kernel) or 2; 0 before the first.  No
  * counterpart in the reference (a profiling aid). */

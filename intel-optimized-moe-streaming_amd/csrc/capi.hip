@@ -578,6 +578,27 @@ int mqh_moe_decode_routed(int gate_type, const void* gate, int up_type, const vo
     return launch_decode(p, s) == hipSuccess ? ST_OK : ST_HIP;
 }
 
+// The same calls with their arguments as 64-bit words, in order (pointers as
+// integers): a foreign-function caller marshals one argument instead of 30.
+int mqh_moe_decode_words(const int64_t* a) {
+    if (!a) return ST_ARG;
+    const auto P = [a](int i) { return (void*)(uintptr_t)a[i]; };
+    return mqh_moe_decode((int)a[0], P(1), (int)a[2], P(3), (int)a[4], P(5), (int)a[6], (int)a[7], (int)a[8], (int)a[9],
+                          P(10), (int)a[11], P(12), (int)a[13], P(14), (int)a[15], (const float*)P(16),
+                          (const float*)P(17), (int)a[18], (const int32_t*)P(19), (const float*)P(20), (int)a[21],
+                          (float*)P(22), (int)a[23], P(24), a[25], P(26));
+}
+
+int mqh_moe_decode_routed_words(const int64_t* a) {
+    if (!a) return ST_ARG;
+    const auto P = [a](int i) { return (void*)(uintptr_t)a[i]; };
+    return mqh_moe_decode_routed((int)a[0], P(1), (int)a[2], P(3), (int)a[4], P(5), (int)a[6], (int)a[7], (int)a[8],
+                                 (int)a[9], P(10), (int)a[11], P(12), (int)a[13], P(14), (int)a[15],
+                                 (const float*)P(16), (const float*)P(17), (int)a[18], (const float*)P(19), (int)a[20],
+                                 (float*)P(21), (int32_t*)P(22), (float*)P(23), (float*)P(24), (int)a[25], P(26), a[27],
+                                 P(28));
+}
+
 int mqh_last_route_kernels(void) { return t_last_route_kernels; }
 
 int64_t mqh_moe_prefill_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate,

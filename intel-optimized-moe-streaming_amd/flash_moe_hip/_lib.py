@@ -29,6 +29,8 @@ EXPORTS = (
     "mqh_moe_decode",
     "mqh_moe_decode_noalloc",
     "mqh_moe_decode_routed",
+    "mqh_moe_decode_words",
+    "mqh_moe_decode_routed_words",
     "mqh_last_route_kernels",
     "mqh_moe_prefill_workspace_bytes",
     "mqh_moe_prefill",
@@ -107,6 +109,9 @@ def _declare(lib: C.CDLL) -> C.CDLL:
         _P, _I, _P, _I64, _P,                    # y, fp16_graph, workspace, ws bytes, stream
     ]
     lib.mqh_moe_decode_routed.restype = _I
+    for f in (lib.mqh_moe_decode_words, lib.mqh_moe_decode_routed_words):
+        f.argtypes = [C.c_char_p]
+        f.restype = _I
     lib.mqh_last_route_kernels.argtypes = []
     lib.mqh_last_route_kernels.restype = _I
     lib.mqh_moe_prefill_workspace_bytes.argtypes = [_I, _I, _I, _I, _I, _I]

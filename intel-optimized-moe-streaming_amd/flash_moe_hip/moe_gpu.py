@@ -15,6 +15,8 @@ reports the faults of the calling thread's calls only.
 """
 from __future__ import annotations
 
+import functools
+import struct
 import threading
 
 import numpy as np
@@ -31,6 +33,34 @@ PREFILL_DOWN_TYPES = PREFILL_TYPES + (8,)
 PREFILL_DIMS = (256, 512, 1024, 2048)
 PREFILL_MAX_EXPERTS = 1024
 Q6_K = 14
+
+# The arguments of mqh_moe_decode and mqh_moe_decode_routed as 64-bit words.
+# A decode call's time on the host is the launches' and this wrapper's: with 27
+# arguments through ctypes, a stream object and a reshape per tensor it took
+# 14.8 us a call (18.5 with its routing and four outputs) where a layer's kernels
+# take 11-14 us; 11.2 (16) so.
+_DECODE_WORDS = struct.Struct("27q")
+_ROUTED_WORDS = struct.Struct("29q")
+
+
+@functools.lru_cache(maxsize=256)
+def _decode_workspace_bytes(lib, n_tokens: int, top_k: int, inter: int, sh_inter: int) -> int:
+    return int(lib.mqh_moe_workspace_bytes(n_tokens, top_k, inter, sh_inter))
+
+
+def _rows(t, n: int, cols: int):
+    """t as [n, cols] (n < 0: as many rows as there are), itself where it has that shape."""
+    s = t.shape
+    return t if len(s) == 2 and s[1] == cols and (n < 0 or s[0] == n) else t.reshape(n, cols)
+
+
+def _shared_words(sh):
+    """The shared expert's eight argument words (types, matrices, size, gate vector)."""
+    if sh is None:
+        return (0, 0, 0, 0, 0, 0, 0, 0)
+    t = sh.types
+    return (t["gate"], sh.gate.data_ptr(), t["up"], sh.up.data_ptr(), t["down"], sh.down.data_ptr(),
+            sh.intermediate, sh.gate_inp.data_ptr() if sh.gate_inp is not None else 0)
 
 
 class MoeRunner:
@@ -91,13 +121,29 @@ class MoeRunner:
         setattr(self._local, "ev_" + slot, ev)
         return [dev[o:o + r.size] for r, o in zip(raws, offs)]
 
-    def _workspace(self, n_tokens: int, top_k: int, inter: int, sh_inter: int, stream):
-        need = int(self.lib.mqh_moe_workspace_bytes(n_tokens, top_k, inter, sh_inter))
+    def _stream(self, stream) -> int:
+        """The handle of `stream`, or of the device's current stream."""
+        import torch
+
+        if stream is not None:
+            return stream.cuda_stream
+        index = self.device.index
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+    def _workspace(self, n_tokens: int, top_k: int, inter: int, sh_inter: int, stream: int, extra: int = 0):
+        """The workspace of a decode call and the address of `extra` bytes after
+        the call's part of it, or 0 where a workspace that is large enough for
+        the call has no room for them (it is not replaced for their sake: that
+        waits for the device, which a call being captured cannot)."""
+        need = _decode_workspace_bytes(self.lib, n_tokens, top_k, inter, sh_inter)
         if need < 0:
             _lib.check(need, "mqh_moe_workspace_bytes")
-        return self._reserve(need, stream)
+        ws = self._ws
+        if ws is None or ws.numel() < need:
+            ws = self._reserve(need + extra, stream)
+        return ws, ws.data_ptr() + need if ws.numel() >= need + extra else 0
 
-    def _reserve(self, need: int, stream):
+    def _reserve(self, need: int, stream: int):
         """The calling thread's workspace, grown to at least `need` bytes.  A
         new buffer is zeroed (its flag words) before it replaces the old one;
         the old one's latched faults are raised first."""
@@ -107,9 +153,9 @@ class MoeRunner:
         if ws is None or need > ws.numel():
             size = max(need, 2 * ws.numel()) if ws is not None else need
             if ws is not None:
-                _lib.check(self.lib.mqh_status(ws.data_ptr(), stream.cuda_stream), "pending kernel")
+                _lib.check(self.lib.mqh_status(ws.data_ptr(), stream), "pending kernel")
             new = torch.empty(size, dtype=torch.uint8, device=self.device)
-            _lib.check(self.lib.mqh_workspace_init(new.data_ptr(), new.numel(), stream.cuda_stream),
+            _lib.check(self.lib.mqh_workspace_init(new.data_ptr(), new.numel(), stream),
                        "mqh_workspace_init")
             self._local.ws = new
             ws = new
@@ -121,38 +167,34 @@ class MoeRunner:
         ids [T,k] int32, weights [T,k] FP32, all CUDA tensors on the layer's device."""
         import torch
 
-        if stream is None:
-            stream = torch.cuda.current_stream(self.device)
-        x = x.reshape(-1, layer.hidden)
+        handle = self._stream(stream)
+        H = layer.hidden
+        x = _rows(x, -1, H)
         T = x.shape[0]
         if x.dtype != torch.float32 or not x.is_contiguous():
             raise ValueError("x must be contiguous FP32")
         top_k = 0 if ids is None else int(ids.shape[-1])
         if top_k:
-            ids = ids.reshape(T, top_k)
-            weights = weights.reshape(T, top_k)
+            ids = _rows(ids, T, top_k)
+            weights = _rows(weights, T, top_k)
             if ids.dtype != torch.int32 or weights.dtype != torch.float32:
                 raise ValueError("ids must be int32 and weights FP32")
             if not (ids.is_contiguous() and weights.is_contiguous()):
                 raise ValueError("ids and weights must be contiguous")
         sh = layer.shared if use_shared else None
         if y is None:
-            y = torch.empty((T, layer.hidden), dtype=torch.float32, device=x.device)
+            y = torch.empty((T, H), dtype=torch.float32, device=x.device)
         if T == 0:
             return y
-        ws = self._workspace(T, top_k, layer.intermediate if top_k else 0, sh.intermediate if sh else 0, stream)
-        t = layer.tensors
-        rc = self.lib.mqh_moe_decode(
-            layer.types["gate"], t["gate"].data_ptr(), layer.types["up"], t["up"].data_ptr(),
-            layer.types["down"], t["down"].data_ptr(), layer.n_experts, layer.hidden, layer.intermediate,
-            sh.types["gate"] if sh else 0, sh.gate.data_ptr() if sh else _NULL,
-            sh.types["up"] if sh else 0, sh.up.data_ptr() if sh else _NULL,
-            sh.types["down"] if sh else 0, sh.down.data_ptr() if sh else _NULL,
-            sh.intermediate if sh else 0,
-            sh.gate_inp.data_ptr() if (sh is not None and sh.gate_inp is not None) else _NULL,
-            x.data_ptr(), T, ids.data_ptr() if top_k else _NULL, weights.data_ptr() if top_k else _NULL, top_k,
-            y.data_ptr(), int(fp16_graph), ws.data_ptr(), ws.numel(), stream.cuda_stream)
-        _lib.check(rc, "mqh_moe_decode")
+        ws, _ = self._workspace(T, top_k, layer.intermediate if top_k else 0, sh.intermediate if sh else 0, handle)
+        t, ty = layer.tensors, layer.types
+        rc = self.lib.mqh_moe_decode_words(_DECODE_WORDS.pack(
+            ty["gate"], t["gate"].data_ptr(), ty["up"], t["up"].data_ptr(), ty["down"], t["down"].data_ptr(),
+            layer.n_experts, H, layer.intermediate, *_shared_words(sh),
+            x.data_ptr(), T, ids.data_ptr() if top_k else 0, weights.data_ptr() if top_k else 0, top_k,
+            y.data_ptr(), int(fp16_graph), ws.data_ptr(), ws.numel(), handle))
+        if rc:
+            _lib.check(rc, "mqh_moe_decode")
         return y
 
     def decode_shared(self, shared, hidden: int, x, *, y=None, stream=None):
@@ -170,7 +212,7 @@ class MoeRunner:
             y = torch.empty((T, hidden), dtype=torch.float32, device=x.device)
         if T == 0:
             return y
-        ws = self._workspace(T, 0, 0, shared.intermediate, stream)
+        ws, _ = self._workspace(T, 0, 0, shared.intermediate, stream.cuda_stream)
         sh = shared
         rc = self.lib.mqh_moe_decode(
             0, _NULL, 0, _NULL, 0, _NULL, 0, hidden, 0,
@@ -220,40 +262,39 @@ class MoeRunner:
         inside the gate/up kernel.  Returns (y, ids, weights)."""
         import torch
 
-        if stream is None:
-            stream = torch.cuda.current_stream(self.device)
+        handle = self._stream(stream)
         w = layer.router_device() if router_w is None else router_w
-        x = x.reshape(-1, layer.hidden)
+        H, E = layer.hidden, layer.n_experts
+        x = _rows(x, -1, H)
         T = x.shape[0]
         if x.dtype != torch.float32 or not x.is_contiguous():
             raise ValueError("x must be contiguous FP32")
-        if w.dtype != torch.float32 or not w.is_contiguous() or tuple(w.shape) != (layer.n_experts, layer.hidden):
-            raise ValueError(f"router weights must be contiguous FP32 [{layer.n_experts}, {layer.hidden}]")
+        if w.dtype != torch.float32 or not w.is_contiguous() or tuple(w.shape) != (E, H):
+            raise ValueError(f"router weights must be contiguous FP32 [{E}, {H}]")
         dev = x.device
         if ids is None:
             ids = torch.empty((T, top_k), dtype=torch.int32, device=dev)
         if weights is None:
             weights = torch.empty((T, top_k), dtype=torch.float32, device=dev)
-        if scores is None:
-            scores = torch.empty((T, layer.n_experts), dtype=torch.float32, device=dev)
         if y is None:
-            y = torch.empty((T, layer.hidden), dtype=torch.float32, device=dev)
+            y = torch.empty((T, H), dtype=torch.float32, device=dev)
         if T == 0:
             return y, ids, weights
         sh = layer.shared if use_shared else None
-        ws = self._workspace(T, top_k, layer.intermediate, sh.intermediate if sh else 0, stream)
-        t = layer.tensors
-        rc = self.lib.mqh_moe_decode_routed(
-            layer.types["gate"], t["gate"].data_ptr(), layer.types["up"], t["up"].data_ptr(),
-            layer.types["down"], t["down"].data_ptr(), layer.n_experts, layer.hidden, layer.intermediate,
-            sh.types["gate"] if sh else 0, sh.gate.data_ptr() if sh else _NULL,
-            sh.types["up"] if sh else 0, sh.up.data_ptr() if sh else _NULL,
-            sh.types["down"] if sh else 0, sh.down.data_ptr() if sh else _NULL,
-            sh.intermediate if sh else 0,
-            sh.gate_inp.data_ptr() if (sh is not None and sh.gate_inp is not None) else _NULL,
-            x.data_ptr(), T, w.data_ptr(), int(top_k), scores.data_ptr(), ids.data_ptr(), weights.data_ptr(),
-            y.data_ptr(), 0, ws.data_ptr(), ws.numel(), stream.cuda_stream)
-        _lib.check(rc, "mqh_moe_decode_routed")
+        # (scores that nobody asked for live in the workspace, as the activations
+        # do, where it has room)
+        ws, scratch = self._workspace(T, top_k, layer.intermediate, sh.intermediate if sh else 0, handle,
+                                      4 * T * E if scores is None else 0)
+        if scores is None and not scratch:
+            scores = torch.empty((T, E), dtype=torch.float32, device=dev)
+        t, ty = layer.tensors, layer.types
+        rc = self.lib.mqh_moe_decode_routed_words(_ROUTED_WORDS.pack(
+            ty["gate"], t["gate"].data_ptr(), ty["up"], t["up"].data_ptr(), ty["down"], t["down"].data_ptr(),
+            E, H, layer.intermediate, *_shared_words(sh),
+            x.data_ptr(), T, w.data_ptr(), int(top_k), scratch if scores is None else scores.data_ptr(),
+            ids.data_ptr(), weights.data_ptr(), y.data_ptr(), 0, ws.data_ptr(), ws.numel(), handle))
+        if rc:
+            _lib.check(rc, "mqh_moe_decode_routed")
         return y, ids, weights
 
     @staticmethod
@@ -309,7 +350,7 @@ class MoeRunner:
                                                            layer.intermediate, int(inside)))
         if need < 0:
             _lib.check(need, "mqh_moe_prefill_workspace_bytes")
-        ws = self._reserve(need, stream)
+        ws = self._reserve(need, stream.cuda_stream)
         t = layer.tensors
         rc = self.lib.mqh_moe_prefill(
             layer.types["gate"], t["gate"].data_ptr(), layer.types["up"], t["up"].data_ptr(),

@@ -106,6 +106,8 @@ class DeltaState:
             if tuple(self.state.shape) != self.shape:
                 raise ValueError("DeltaNet state shape mismatch")
         self._flags = torch.zeros(64, dtype=torch.int32, device=self.state.device)
+        nv, dv, dk = self.shape
+        self._in_shapes = [(nv, dk), (nv, dk), (nv, dv), (nv,), (nv,)]
 
     def reset(self):
         self.state.zero_()
@@ -114,17 +116,18 @@ class DeltaState:
         import torch
 
         nv, dv, dk = self.shape
-        args = [q, k, v, beta, gate]
-        shapes = [(nv, dk), (nv, dk), (nv, dv), (nv,), (nv,)]
-        for a, shp in zip(args, shapes):
-            if a.dtype != torch.float32 or not a.is_contiguous() or tuple(a.shape) != shp:
-                raise ValueError(f"DeltaNet inputs must be contiguous FP32 of shapes {shapes}")
+        f32 = torch.float32
+        for a, shp in zip((q, k, v, beta, gate), self._in_shapes):
+            if a.dtype != f32 or a.shape != shp or not a.is_contiguous():
+                raise ValueError(f"DeltaNet inputs must be contiguous FP32 of shapes {self._in_shapes}")
+        state = self.state
         if out is None:
-            out = torch.empty((nv, dv), dtype=torch.float32, device=self.state.device)
-        if stream is None:
-            stream = torch.cuda.current_stream(self.state.device)
-        rc = self.lib.mqh_delta_heads(self.state.data_ptr(), *[a.data_ptr() for a in args], out.data_ptr(),
-                                      nv, dk, dv, self._flags.data_ptr(), stream.cuda_stream)
+            out = torch.empty((nv, dv), dtype=f32, device=state.device)
+        # (the current stream's handle without a stream object: a step is shorter
+        # than this wrapper)
+        handle = stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(state.get_device())
+        rc = self.lib.mqh_delta_heads(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
+                                      gate.data_ptr(), out.data_ptr(), nv, dk, dv, self._flags.data_ptr(), handle)
         _lib.check(rc, "mqh_delta_heads")
         return out
 

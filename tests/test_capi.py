@@ -153,3 +153,35 @@ def test_iq4_nl_stays_outside_the_reference_contracts(lib):
     buf = np.zeros(18, np.uint8)
     out = np.zeros(32, np.float32)
     assert lib.dequant_k(20, buf.ctypes.data, out.ctypes.data, 32, 0) == -1
+
+
+def test_word_calls_take_the_same_arguments(lib):
+    """The calls with their arguments as 64-bit words validate as the plain ones
+    do: each word reaches its argument (host-side statuses, no kernel runs)."""
+    import struct
+
+    bufs = [np.zeros(1 << 16, np.uint8) for _ in range(12)]
+    p = [b.ctypes.data + (-b.ctypes.data) % 256 for b in bufs]
+
+    def decode(**kw):
+        a = dict(gt=12, g=p[0], ut=12, u=p[1], dt=14, d=p[2], E=4, H=256, I=256, sgt=12, sg=p[3], sut=12, su=p[4],
+                 sdt=14, sd=p[5], sI=256, sgi=p[6], x=p[7], T=1, ids=p[8], w=p[9], k=2, y=p[10], f=0, ws=p[11], wb=0,
+                 st=0)
+        a.update(kw)
+        v = list(a.values())
+        plain = lib.mqh_moe_decode(*[None if i in (1, 3, 5, 10, 12, 14, 16, 17, 19, 20, 22, 24) and q == 0 else q
+                                     for i, q in enumerate(v)])
+        assert lib.mqh_moe_decode_words(struct.pack("27q", *v)) == plain, kw
+        r = v[:18] + [v[18], p[9], v[21], p[6], v[19], v[20], v[22], v[23], v[24], v[25], v[26]]
+        plain_r = lib.mqh_moe_decode_routed(*[None if i in (1, 3, 5, 10, 12, 14, 16, 17, 22, 23, 24, 26) and q == 0
+                                              else q for i, q in enumerate(r)])
+        assert lib.mqh_moe_decode_routed_words(struct.pack("29q", *r)) == plain_r, kw
+        return plain
+
+    assert decode() == -6   # every argument is right but the workspace's size
+    assert decode(gt=99) == -2 and decode(ut=99) == -2 and decode(dt=99) == -2 and decode(sdt=99) == -2
+    for name in ("g", "u", "d", "su", "sd", "x", "ids", "w", "y", "ws"):
+        assert decode(**{name: 0}) == -1, name
+    assert decode(H=100) == -2 and decode(I=100) == -2 and decode(sI=100) == -2 and decode(E=0) == -1
+    assert decode(T=0) == -1 and decode(k=65) == -1 and decode(f=2) == -1 and decode(g=p[0] + 1) == -1
+    assert lib.mqh_moe_decode_words(None) == -1 and lib.mqh_moe_decode_routed_words(None) == -1

@@ -271,3 +271,41 @@ def test_route_scores_many_tokens(T, H, E, k):
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     bound = H * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
     assert np.all(np.abs(scores - x64 @ w64) <= bound)
+
+
+def test_routed_scores_in_and_out_of_the_workspace():
+    """Routed decode gives the same bits with its scores in the caller's tensor,
+    in the workspace (a runner's first call makes room for them) and, where a
+    plain decode call made the workspace without it, in a tensor of their own --
+    there also under capture, without the workspace being replaced."""
+    import torch
+    from flash_moe_hip.moe_gpu import MoeRunner
+
+    from test_gpu_decode import make_layer
+
+    t = {"gate": 12, "up": 12, "down": 14}
+    layer, _, _ = make_layer(91, 16, 512, 256, t, shared_types=t)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(2, 512, generator=g, device="cuda")
+    w = torch.randn(16, 512, generator=g, device="cuda") * 0.05
+    own = torch.empty(2, 16, device="cuda")
+    print("routed scores in and out of the workspace", flush=True)
+    want, ids, weights = MoeRunner().decode_routed(layer, x, 4, router_w=w, scores=own)
+    first = MoeRunner().decode_routed(layer, x, 4, router_w=w)
+    runner = MoeRunner()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        runner.decode(layer, x, ids, weights)
+    torch.cuda.synchronize()
+    ws = runner._ws
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got = runner.decode_routed(layer, x, 4, router_w=w)
+    assert runner._ws is ws
+    for _ in range(3):
+        got[0].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b, c in zip((want, ids, weights), first, got):
+            assert torch.equal(a, b) and torch.equal(a, c)
