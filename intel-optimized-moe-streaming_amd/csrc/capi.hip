@@ -606,10 +606,11 @@ int64_t mqh_moe_prefill_workspace_bytes(int n_tokens, int top_k, int n_experts, 
     if (n_tokens <= 0 || top_k < 0 || top_k > 64 || n_experts <= 0 || hidden <= 0 || intermediate <= 0 ||
         (has_shared != 0 && has_shared != 1) || (top_k == 0 && !has_shared))
         return ST_ARG;
-    // (the types are not known here: room for either tile width)
-    int64_t need = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, false).total;
-    if (prefill_wide_size(n_tokens, top_k, n_experts, hidden, intermediate, has_shared))
-        need = std::max(need, prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, true).total);
+    // room for either tile width whatever the size (the types are not known
+    // here, and a workspace for a prompt has to do for every shorter one)
+    const int64_t need =
+        std::max(prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, false).total,
+                 prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, true).total);
     return need;
 }
 

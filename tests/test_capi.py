@@ -185,3 +185,14 @@ def test_word_calls_take_the_same_arguments(lib):
     assert decode(H=100) == -2 and decode(I=100) == -2 and decode(sI=100) == -2 and decode(E=0) == -1
     assert decode(T=0) == -1 and decode(k=65) == -1 and decode(f=2) == -1 and decode(g=p[0] + 1) == -1
     assert lib.mqh_moe_decode_words(None) == -1 and lib.mqh_moe_decode_routed_words(None) == -1
+
+
+def test_prefill_workspace_does_for_every_shorter_prompt(lib):
+    """The workspace of a prompt is at least that of any shorter one, across the
+    sizes at which the tile width changes (4096 pairs, 32 tokens an expert, and
+    2^32 plane values, past which the 16-token tiles are back)."""
+    for k, E, H, I, sh in ((8, 256, 2048, 512, 1), (2, 8, 256, 2048, 0), (8, 60, 512, 256, 1), (0, 1, 2048, 1024, 1)):
+        sizes = sorted({1, 2, 15, 16, 17, 60, 127, 128, 455, 456, 512, 913, 914, 1027, 2048, 4096, 8192, 65535, 200000,
+                        233016, 233017, 233018, 262144, 524288, 1048576, 2097152, 2200000})
+        need = [lib.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, sh) for T in sizes]
+        assert need[0] > 0 and all(a <= b for a, b in zip(need, need[1:])), (k, E, H, I, sh)
