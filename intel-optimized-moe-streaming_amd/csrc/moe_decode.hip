@@ -161,10 +161,13 @@ __global__ __launch_bounds__(64 * GEN_WAVES_A) void k_gate_up(DecodeParams p) {
     __asm__ volatile("" ::"s"(id), "s"(gate), "s"(up), "s"(sh_gate), "s"(sh_up), "s"(geb), "s"(ueb), "s"(gtr), "s"(utr),
                      "s"(gts), "s"(uts), "s"(ir), "s"(is));
     const int I = shared ? is : ir, gt = shared ? gts : gtr, ut = shared ? uts : utr;
-    if (id < 0 || (!shared && id >= p.n_experts)) {
-        // Out-of-range expert id: flag it and contribute nothing.
-        if (threadIdx.x == 0 && blockIdx.x == 0) atomicOr(&p.flags[FLAG_BAD_ID], 1);
-        if (r < I && lp == 0) at[r] = 0.0f;
+    // nothing to do for a wave whose rows are all past this slot's intermediate
+    // size (the grid is the larger one's, routed or shared), and for an expert id
+    // out of range, which is flagged and contributes nothing
+    const bool bad = id < 0 || (!shared && id >= p.n_experts);
+    if (bad || (int)(blockIdx.x * GEN_WAVES_A + __builtin_amdgcn_readfirstlane(wave)) * rpw >= I) {
+        if (bad && threadIdx.x == 0 && blockIdx.x == 0) atomicOr(&p.flags[FLAG_BAD_ID], 1);
+        if (bad && r < I && lp == 0) at[r] = 0.0f;
         return;
     }
     const uint8_t* G = shared ? sh_gate : gate + (int64_t)id * geb;

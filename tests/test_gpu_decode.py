@@ -706,3 +706,42 @@ def test_generic_sizes(hip, oracle_mod, gt, ut, dt, H, I, sh_I, k, T):
         if half is not None:
             want16 = oracle_layer(oracle_mod, layer, host, shared, X[tok], ids[tok].tolist(), ws[tok].tolist(), fp16=1)
             assert oracle_mod.max_relative_error(half[tok], want16) <= TOL, tok
+
+
+def test_generic_sizes_cost_no_more_than_their_slots(hip):
+    """A slot's rows in kernel A are its own expert's, not the largest slot's: a
+    call of eight routed experts and a shared one sixteen times their size takes
+    1.7 times its routed and its shared part (kernel B's longest wave is the
+    shared expert's), and took four times them with every slot at the shared
+    expert's rows."""
+    import torch
+
+    from flash_moe_hip.layer_store import ExpertLayer
+    from flash_moe_hip.moe_gpu import MoeRunner
+
+    t = {"gate": 12, "up": 12, "down": 14}
+    E, H, I, k, T = 16, 1536, 512, 8, 16
+    layer = ExpertLayer.synthetic(t, E, H, I, seed=5, shared_types=t, shared_intermediate=16 * I, scale=0.001)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(T, H, generator=g, device="cuda")
+    top = torch.topk(torch.randn(T, E, generator=g, device="cuda"), k, dim=1)
+    ids, w = top.indices.int().contiguous(), torch.softmax(top.values, dim=1).contiguous()
+    runner = MoeRunner()
+    print("generic sizes: time of a call against its parts", flush=True)
+
+    def us(*args, **kw):
+        times = []
+        for _ in range(9):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                runner.decode(layer, x, *args, **kw)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 200)
+        return sorted(times)[4]
+
+    both, routed, shared = us(ids, w), us(ids, w, use_shared=False), us(None, None)
+    assert hip.mqh_last_decode_path() == 1
+    print(f"both {both:.1f} us, routed {routed:.1f}, shared {shared:.1f}", flush=True)
+    assert both <= 2.5 * (routed + shared)
