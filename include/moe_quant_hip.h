@@ -216,7 +216,9 @@ int mqh_delta_heads(float* state, const float* q, const float* k, const float* v
                     const float* gate, float* output, int heads, int key_dim, int value_dim, void* workspace,
                     void* stream);
 
-/* Bytes of workspace mqh_moe_prefill needs (has_shared: 0 or 1). */
+/* Bytes of workspace for mqh_moe_prefill (has_shared: 0 or 1): what the tile
+ * width chosen for the prompt needs.  A workspace that only has room for
+ * 16-token tiles is accepted as well, and they are used. */
 int64_t mqh_moe_prefill_workspace_bytes(int n_tokens, int top_k, int n_experts, int hidden, int intermediate,
                                         int has_shared);
 
@@ -244,6 +246,11 @@ int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up
                     int sh_down_type, const void* sh_down, int sh_intermediate, const float* sh_gate_inp,
                     const void* x, int x_bf16, int n_tokens, const int32_t* ids, const float* weights,
                     int top_k, float* y, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Tokens per tile of the calling thread's last mqh_moe_prefill: 16 or 64 (the
+ * same results); 0 before the first.  No counterpart in the reference (a
+ * profiling aid). */
+int mqh_last_prefill_tile(void);
 
 /* Select the kernels behind mqh_moe_decode and moe_quant_expert: 0 (default)
  * = the two integer-digit fast kernels (gate/up + SwiGLU, then down +

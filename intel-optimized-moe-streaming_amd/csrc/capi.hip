@@ -38,6 +38,8 @@ thread_local int t_last_path = -1;
 // router kernels of this thread's last routed decode (1: the select step ran
 // inside the gate/up kernel, 2: a select kernel of its own)
 thread_local int t_last_route_kernels = 0;
+// tile width of this thread's last prefill
+thread_local int t_last_prefill_tile = 0;
 
 hipError_t launch_decode(const DecodeParams& p, hipStream_t s) {
     const KernelEvents ev = t_events;
@@ -646,8 +648,12 @@ int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up
     if (!prefill_supported(p)) return ST_TYPE;
     const bool wide = prefill_wide_types(down_type, has_shared, sh_down_type) &&
                       prefill_wide_size(n_tokens, top_k, n_experts, hidden, intermediate, has_shared);
-    const PrefillLayout L = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, wide);
+    PrefillLayout L = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, wide);
+    // (16-token tiles give the same bits in a smaller workspace)
+    if (workspace_bytes < L.total && wide)
+        L = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, false);
     if (workspace_bytes < L.total) return ST_WORKSPACE;
+    t_last_prefill_tile = L.tile;
 
     uint8_t* WS = (uint8_t*)workspace;
     p.sh_gate = (const uint8_t*)sh_gate; p.sh_up = (const uint8_t*)sh_up; p.sh_down = (const uint8_t*)sh_down;
@@ -668,6 +674,8 @@ int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up
     t_events = KernelEvents();
     return launch_prefill(p, (hipStream_t)stream, ev) == hipSuccess ? ST_OK : ST_HIP;
 }
+
+int mqh_last_prefill_tile(void) { return t_last_prefill_tile; }
 
 int mqh_profile_next_decode(void* a_start, void* a_stop, void* b_start, void* b_stop) {
     t_events.a_start = (hipEvent_t)a_start;

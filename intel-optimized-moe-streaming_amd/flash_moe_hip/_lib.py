@@ -34,6 +34,7 @@ EXPORTS = (
     "mqh_last_route_kernels",
     "mqh_moe_prefill_workspace_bytes",
     "mqh_moe_prefill",
+    "mqh_last_prefill_tile",
     "mqh_set_decode_path",
     "mqh_last_decode_kernels",
     "mqh_last_decode_path",
@@ -114,6 +115,8 @@ def _declare(lib: C.CDLL) -> C.CDLL:
         f.restype = _I
     lib.mqh_last_route_kernels.argtypes = []
     lib.mqh_last_route_kernels.restype = _I
+    lib.mqh_last_prefill_tile.argtypes = []
+    lib.mqh_last_prefill_tile.restype = _I
     lib.mqh_moe_prefill_workspace_bytes.argtypes = [_I, _I, _I, _I, _I, _I]
     lib.mqh_moe_prefill_workspace_bytes.restype = _I64
     lib.mqh_moe_prefill.argtypes = [

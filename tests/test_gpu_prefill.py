@@ -339,3 +339,55 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     check(oracle_mod, layer, host, shared, X[T:T + 9], ids[T:T + 9], ws[T:T + 9], got[T:T + 9], "expert 7")
     for r in range(2, reps):
         np.testing.assert_array_equal(got[r * T:(r + 1) * T], got[T:2 * T])
+
+
+def workspace_16(T, k, E, H, I, has_shared):
+    """Bytes the kernels of 16-token tiles need: flags, per-token gates, tile
+    records and their columns, activations and pair outputs, token planes."""
+    def up(n):
+        return (n + 255) // 256 * 256
+
+    S = k + has_shared
+    tiles = max(min(E, T * k) + -(-T * k // 16) + (-(-T // 16) if has_shared else 0), 1)
+    return (256 + up(4 * T) + up(16 * tiles) + 256 + 2 * up(64 * tiles) + up(4 * T * S * I) + up(4 * T * S * H)
+            + 2 * up(2 * T * H) + up(T * (H // 32) * 4) + up(4 * T))
+
+
+def test_prefill_in_a_16_token_workspace(hip):
+    """A prompt whose size is the 64-token tiles' runs in a workspace that only
+    has room for 16-token tiles, on those, with the same bits; one byte less is
+    refused."""
+    import torch
+
+    from flash_moe_hip.layer_store import ExpertLayer
+    from flash_moe_hip.moe_gpu import MoeRunner
+
+    t = {"gate": 12, "up": 12, "down": 14}
+    T, k, E, H, I = 1100, 4, 8, 2048, 512
+    layer = ExpertLayer.synthetic(t, E, H, I, seed=9, shared_types=t)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn(T, H, generator=g, device="cuda")
+    top = torch.topk(torch.randn(T, E, generator=g, device="cuda"), k, dim=1)
+    ids, w = top.indices.int().contiguous(), torch.softmax(top.values, dim=1).contiguous()
+    print("prefill in a 16-token workspace", flush=True)
+    want = MoeRunner().prefill(layer, x, ids, w)
+    assert hip.mqh_last_prefill_tile() == 64
+    need = workspace_16(T, k, E, H, I, 1)
+    assert need < hip.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, 1)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert hip.mqh_workspace_init(ws.data_ptr(), need, stream) == 0
+    y = torch.empty(T, H, device="cuda")
+    sh, d = layer.shared, layer.tensors
+
+    def call(nbytes):
+        return hip.mqh_moe_prefill(
+            12, d["gate"].data_ptr(), 12, d["up"].data_ptr(), 14, d["down"].data_ptr(), E, H, I,
+            12, sh.gate.data_ptr(), 12, sh.up.data_ptr(), 14, sh.down.data_ptr(), I, sh.gate_inp.data_ptr(),
+            x.data_ptr(), 0, T, ids.data_ptr(), w.data_ptr(), k, y.data_ptr(), ws.data_ptr(), nbytes, stream)
+
+    assert call(need - 1) == -6
+    assert call(need) == 0
+    assert hip.mqh_last_prefill_tile() == 16
+    assert hip.mqh_status(ws.data_ptr(), stream) == 0
+    assert torch.equal(y, want)
