@@ -647,7 +647,8 @@ int mqh_moe_prefill(int gate_type, const void* gate, int up_type, const void* up
     p.sh_gate_type = sh_gate_type; p.sh_up_type = sh_up_type; p.sh_down_type = sh_down_type;
     if (!prefill_supported(p)) return ST_TYPE;
     const bool wide = prefill_wide_types(down_type, has_shared, sh_down_type) &&
-                      prefill_wide_size(n_tokens, top_k, n_experts, hidden, intermediate, has_shared);
+                      prefill_wide_size(n_tokens, top_k, n_experts, hidden, intermediate, has_shared,
+                                        top_k > 0 ? gate_type : sh_gate_type);
     PrefillLayout L = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, wide);
     // (16-token tiles give the same bits in a smaller workspace)
     if (workspace_bytes < L.total && wide)

@@ -143,8 +143,9 @@ struct PrefillLayout {
     int max_tiles, tile;
 };
 
-// Whether a prompt's size, and a layer's types, are the wide tiles'
-bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared);
+// Whether a prompt's size (for a gate type), and a layer's down types, are the
+// wide tiles'
+bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, int gate_type);
 bool prefill_wide_types(int down_type, int has_shared, int sh_down_type);
 PrefillLayout prefill_layout(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, bool wide);
 bool prefill_supported(const PrefillParams& p);

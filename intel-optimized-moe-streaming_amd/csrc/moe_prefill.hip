@@ -27,6 +27,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "kquant_frag.h"
 #include "moe_decode.h"
@@ -94,14 +95,48 @@ constexpr int pf_occupancy(int lds_bytes) {
 
 // Tiles of PREFILL_WIDE tokens (moe_prefill_wide.hip) from PF_WIDE_TOKENS
 // (token, slot) pairs per expert on average (the shared expert counts as one),
-// and PF_WIDE_PAIRS in all.  Layer times in us, 64-token and 16-token tiles:
-//   Q4_K/Q6_K, BF16  18 an expert 303/298, 36 366/423, 72 555/715
-//   Q3_K, FP32       18 310/286, 36 399/468, 72 596/791
-//   Q5_K, FP32       16 275/258, 32 326/405, 64 514/689
-//   Q6_K, FP32       18 433/396, 36 538/601, 72 836/1078
-// and with few experts too few workgroups: 256 tokens of 16 experts (2304
-// pairs) 126/120 in Q3_K, 512 of 60 (4608) 205/208.
+// PF_WIDE_PAIRS in all, and an amount of work: the wide tiles save building the
+// weight operands again for every 16 tokens (most in Q6_K, least in Q4_K) and
+// pay for it with few, long workgroups (128 x 64 or 256 x 64 outputs, one or two
+// a CU, 256 columns a stage) and the pass that makes the activation planes, so
+// they need the more of it the smaller the matrices are.  The amount is
+// pairs sqrt(pairs per expert) hidden inter, or without the matrix size at
+// hidden 256, whose down projection has one workgroup a tile.
+//
+// Layer times in us, 64-token and 16-token tiles, BF16 tokens of 128 or 256
+// experts, top-8 (Q4_K/Q6_K with a shared expert, Q3_K with one in Q6_K):
+//   hidden x inter     2048x512           1024x256          512x512           512x256
+//   pairs (an expert)
+//   Q4_K/Q6_K
+//      6192   (48)   241/251 (1.1)     104/89  (.28)     102/82  (.28)      76/61  (.14)
+//     16452   (64)   495/616 (3.5)     181/199 (.86)     175/180 (.86)     123/122 (.43)
+//     32904  (128)   852/1174 (9.8)    331/376 (2.4)     312/332 (2.4)     201/218 (1.2)
+//   Q5_K
+//      6144   (48)   213/239 (1.5)      71/85  (.37)      90/79  (.37)      67/57  (.19)
+//     16384   (64)   425/605 (4.6)     161/184 (1.1)     163/171 (1.1)     110/118 (.57)
+//   Q3_K
+//      4131   (32)   199/197 (2.0)      90/79  (.51)      81/80  (.51)      64/57  (.25)
+//      8262   (64)   249/339 (5.8)     109/128 (1.5)     104/128 (1.5)      77/86  (.72)
+//   Q6_K
+//      4096   (32)   259/276 (3.4)      91/99  (.87)      90/109 (.87)      61/71  (.43)
+//      8192   (64)   399/472 (9.9)     158/171 (2.4)     143/183 (2.4)     105/113 (1.2)
+// (in parentheses the amount over the type's threshold).  Hidden 256, inter 512,
+// 65536 pairs, 256 an expert: 403/349 in Q4_K, 374/338 in Q5_K, 397/441 in Q3_K,
+// 545/558 in Q6_K; 8192 pairs, 32 an expert: 96/67, 75/66, 93/81, 110/100.  Half
+// as wide a matrix needs twice the pairs (gate/up has pairs inter / 8192
+// workgroups, one a CU from there on): 4131 pairs of hidden 2048, inter 256 in
+// Q6_K with a shared expert take 22 % longer in 64-token tiles.
+// Below PF_WIDE_TOKENS (hidden 2048, inter 512, 18 and 36 pairs an expert):
+// Q4_K/Q6_K 303/298 and 366/423, Q3_K 310/286 and 399/468, Q6_K 433/396 and
+// 538/601; Q5_K, 16 and 32 an expert, 275/258 and 326/405.  Below PF_WIDE_PAIRS
+// it depends on the type (256 tokens of 16 experts, 2304 pairs: 126/120 in Q3_K,
+// 93/101 in Q4_K, 88/94 in Q5_K, 133/152 in Q6_K); the line is the slowest type's.
 constexpr int64_t PF_WIDE_TOKENS = 32, PF_WIDE_PAIRS = 4096;
+static double pf_wide_work(int gate_type, int hidden) {
+    const bool q36 = gate_type == T_Q3_K || gate_type == T_Q6_K;
+    if (hidden == 256) return q36 ? 4e5 : 2e6;
+    return gate_type == T_Q6_K ? 7e9 : gate_type == T_Q3_K ? 1.2e10 : gate_type == T_Q5_K ? 3e10 : 4e10;
+}
 
 #ifndef PF_OCC_GU
 #define PF_OCC_GU
@@ -783,11 +818,14 @@ bool prefill_supported(const PrefillParams& p) {
     return true;
 }
 
-bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared) {
+bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, int gate_type) {
     const int64_t P = (int64_t)n_tokens * (top_k + (has_shared ? 1 : 0));
+    const int64_t experts = (top_k > 0 ? n_experts : 0) + (has_shared ? 1 : 0);
     // (the wide kernels' row offsets into the planes are 32 bits)
-    return P >= PF_WIDE_TOKENS * ((top_k > 0 ? n_experts : 0) + (has_shared ? 1 : 0)) && P >= PF_WIDE_PAIRS &&
-           P * std::max(hidden, inter) < ((int64_t)1 << 32);
+    if (P < PF_WIDE_TOKENS * experts || P < PF_WIDE_PAIRS || P * inter < PF_WIDE_PAIRS * 512 ||
+        P * std::max(hidden, inter) >= ((int64_t)1 << 32)) return false;
+    const double work = (double)P * std::sqrt((double)P / (double)experts);
+    return work * (hidden == 256 ? 1.0 : (double)hidden * inter) >= pf_wide_work(gate_type, hidden);
 }
 
 bool prefill_wide_types(int down_type, int has_shared, int sh_down_type) {

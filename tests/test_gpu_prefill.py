@@ -322,7 +322,7 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     first = rng.permutation(first)
     # the repetitions' second pairs go to expert 0 and theirs, too, to 7: the
     # other experts keep the counts above
-    reps = 4096 // (T * 2) + 1
+    reps = 100 if H == 256 else 13
     X1 = rng.standard_normal((T, H)).astype(np.float32) * rng.uniform(0.01, 30, (T, 1)).astype(np.float32)
     X = np.concatenate([X1] * reps)
     ids = np.zeros((T * reps, 2), np.int64)
@@ -335,6 +335,7 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     print(f"prefill wide tiles types={types} shared={sh} H={H} I={I} T={len(X)} bf16={x_bf16}", flush=True)
     got, status = run_prefill(layer, X, ids, ws, x_bf16=x_bf16)
     assert status == 0
+    assert hip.mqh_last_prefill_tile() == (16 if dt == 8 else 64)
     check(oracle_mod, layer, host, shared, X[:T], ids[:T], ws[:T], got[:T], f"wide {types} {shape}")
     check(oracle_mod, layer, host, shared, X[T:T + 9], ids[T:T + 9], ws[T:T + 9], got[T:T + 9], "expert 7")
     for r in range(2, reps):
@@ -391,3 +392,47 @@ def test_prefill_in_a_16_token_workspace(hip):
     assert hip.mqh_last_prefill_tile() == 16
     assert hip.mqh_status(ws.data_ptr(), stream) == 0
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("types,sh,shape,E,k,T,tile", [
+    # (hidden 2048 and 256, either side of the pairs an expert and of the amount of work)
+    ((12, 14), True, (2048, 512), 256, 8, 4096, 64),
+    ((12, 14), True, (2048, 512), 256, 8, 909, 16),
+    ((12, 14), True, (256, 512), 256, 8, 914, 16),
+    ((13, 13), False, (256, 2048), 8, 2, 4096, 16),
+    ((12, 14), True, (256, 256), 1, 0, 4096, 16),
+    ((11, 11), True, (256, 512), 16, 8, 4096, 64),
+    # amounts of work of each type
+    ((12, 14), True, (512, 256), 60, 4, 1640, 16),
+    ((12, 14), True, (1024, 512), 8, 2, 2048, 64),
+    ((13, 13), False, (512, 512), 60, 8, 768, 16),
+    ((13, 13), False, (512, 512), 60, 8, 1536, 64),
+    ((11, 11), False, (512, 256), 60, 8, 520, 16),
+    ((11, 11), False, (512, 512), 60, 8, 768, 64),
+    ((14, 14), False, (512, 256), 60, 8, 600, 16),
+    ((14, 14), False, (512, 256), 60, 8, 1024, 64),
+    # one super-block of intermediate: twice the pairs
+    ((14, 14), False, (2048, 256), 128, 8, 512, 16),
+    ((14, 14), False, (2048, 256), 128, 8, 1024, 64),
+    ((12, 8), False, (2048, 512), 8, 2, 4096, 16),
+])
+def test_prefill_tile_width(hip, types, sh, shape, E, k, T, tile):
+    """The tile width of a prompt follows the matrix size and type as well as its
+    length: where the 64-token tiles measured slower the 16-token ones run."""
+    import torch
+
+    from flash_moe_hip.layer_store import ExpertLayer
+    from flash_moe_hip.moe_gpu import MoeRunner
+
+    (gt, dt), (H, I) = types, shape
+    t = {"gate": gt, "up": gt, "down": dt}
+    layer = ExpertLayer.synthetic(t, E, H, I, seed=T, shared_types=t if sh else None)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, H, generator=g, device="cuda").to(torch.bfloat16)
+    top = torch.topk(torch.randn(T, E, generator=g, device="cuda"), k, dim=1)
+    ids, w = top.indices.int().contiguous(), torch.softmax(top.values, dim=1).contiguous()
+    print(f"prefill tile width {types} H={H} I={I} E={E} k={k} T={T}", flush=True)
+    runner = MoeRunner()
+    y = runner.prefill(layer, x, ids, w)
+    assert runner.status() == 0 and bool(torch.isfinite(y).all())
+    assert hip.mqh_last_prefill_tile() == tile
