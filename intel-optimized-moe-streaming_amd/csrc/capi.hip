@@ -608,11 +608,15 @@ int64_t mqh_moe_prefill_workspace_bytes(int n_tokens, int top_k, int n_experts, 
     if (n_tokens <= 0 || top_k < 0 || top_k > 64 || n_experts <= 0 || hidden <= 0 || intermediate <= 0 ||
         (has_shared != 0 && has_shared != 1) || (top_k == 0 && !has_shared))
         return ST_ARG;
-    // room for either tile width whatever the size (the types are not known
-    // here, and a workspace for a prompt has to do for every shorter one)
-    const int64_t need =
-        std::max(prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, false).total,
-                 prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, true).total);
+    // The tile width follows the gate type, which is not known here: room for 64
+    // tokens where Q6_K, the first to take them, does.  Past the last size of
+    // theirs, room for that one: a workspace for a prompt does for every shorter
+    // one without a change of width.
+    int64_t need = prefill_layout(n_tokens, top_k, n_experts, hidden, intermediate, has_shared, false).total;
+    const int wide = std::min(n_tokens, prefill_wide_max_tokens(top_k + has_shared, hidden, intermediate));
+    if (prefill_wide_size(wide, top_k, n_experts, hidden, intermediate, has_shared, T_Q6_K))
+        need = std::max(need,
+                        prefill_layout(wide, top_k, n_experts, hidden, intermediate, has_shared, true).total);
     return need;
 }
 

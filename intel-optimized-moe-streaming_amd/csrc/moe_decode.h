@@ -143,6 +143,8 @@ struct PrefillLayout {
     int max_tiles, tile;
 };
 
+// Most tokens of a prompt on the wide tiles
+int prefill_wide_max_tokens(int slots, int hidden, int inter);
 // Whether a prompt's size (for a gate type), and a layer's down types, are the
 // wide tiles'
 bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, int gate_type);

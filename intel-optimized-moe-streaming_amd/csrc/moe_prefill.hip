@@ -818,12 +818,17 @@ bool prefill_supported(const PrefillParams& p) {
     return true;
 }
 
+// (the wide kernels' row offsets into the planes are 32 bits)
+int prefill_wide_max_tokens(int slots, int hidden, int inter) {
+    return (int)(((((int64_t)1 << 32) - 1) / std::max(hidden, inter)) / slots);
+}
+
 bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, int gate_type) {
     const int64_t P = (int64_t)n_tokens * (top_k + (has_shared ? 1 : 0));
     const int64_t experts = (top_k > 0 ? n_experts : 0) + (has_shared ? 1 : 0);
-    // (the wide kernels' row offsets into the planes are 32 bits)
     if (P < PF_WIDE_TOKENS * experts || P < PF_WIDE_PAIRS || P * inter < PF_WIDE_PAIRS * 512 ||
-        P * std::max(hidden, inter) >= ((int64_t)1 << 32)) return false;
+        n_tokens > prefill_wide_max_tokens(top_k + (has_shared ? 1 : 0), hidden, inter))
+        return false;
     const double work = (double)P * std::sqrt((double)P / (double)experts);
     return work * (hidden == 256 ? 1.0 : (double)hidden * inter) >= pf_wide_work(gate_type, hidden);
 }

@@ -196,3 +196,39 @@ def test_prefill_workspace_does_for_every_shorter_prompt(lib):
                         233016, 233017, 233018, 262144, 524288, 1048576, 2097152, 2200000})
         need = [lib.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, sh) for T in sizes]
         assert need[0] > 0 and all(a <= b for a, b in zip(need, need[1:])), (k, E, H, I, sh)
+
+
+def workspace_16(T, k, E, H, I, has_shared):
+    """Bytes the prefill kernels of 16-token tiles need: flags, per-token gates,
+    tile records and their columns, activations and pair outputs, token planes."""
+    def up(n):
+        return (n + 255) // 256 * 256
+
+    S = k + has_shared
+    tiles = max(min(E, T * k) + -(-T * k // 16) + (-(-T // 16) if has_shared else 0), 1)
+    return (256 + up(4 * T) + up(16 * tiles) + 256 + 2 * up(64 * tiles) + up(4 * T * S * I) + up(4 * T * S * H)
+            + 2 * up(2 * T * H) + up(T * (H // 32) * 4) + up(4 * T))
+
+
+@pytest.mark.parametrize("k,E,H,I,sh,last", [
+    (8, 256, 2048, 512, 1, 913),      # 32 pairs an expert
+    (8, 60, 512, 256, 1, 910),        # one gate/up workgroup a CU
+    (8, 8, 2048, 2048, 0, 511),       # 4096 pairs
+    (2, 8, 256, 2048, 0, 5428),       # pairs sqrt(pairs an expert)
+])
+def test_prefill_workspace_of_prompts_below_the_wide_tiles(lib, k, E, H, I, sh, last):
+    """Only prompts that some type takes 64-token tiles for pay for their planes."""
+    for T in (1, 3, last // 2, last):
+        assert lib.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, sh) == workspace_16(T, k, E, H, I, sh), T
+    T, S = last + 1, k + sh
+    planes = T * S * (4 * I + 4 * (I // 32) + 4)
+    assert lib.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, sh) >= workspace_16(T, k, E, H, I, sh) + planes // 2
+
+
+def test_prefill_workspace_past_the_wide_tiles(lib):
+    """A prompt of 2^32 plane values or more has room for the longest one below."""
+    k, E, H, I, sh = 8, 256, 2048, 512, 1
+    last = (2 ** 32 - 1) // H // (k + sh)
+    need = [lib.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, sh) for T in (last, last + 1, 2 * last)]
+    assert need[1] == need[0] > workspace_16(last + 1, k, E, H, I, sh)
+    assert need[2] == workspace_16(2 * last, k, E, H, I, sh)

@@ -11,6 +11,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from test_capi import workspace_16
 from test_gpu_decode import host_expert, make_layer, oracle_layer
 
 pytestmark = pytest.mark.gpu
@@ -340,18 +341,6 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     check(oracle_mod, layer, host, shared, X[T:T + 9], ids[T:T + 9], ws[T:T + 9], got[T:T + 9], "expert 7")
     for r in range(2, reps):
         np.testing.assert_array_equal(got[r * T:(r + 1) * T], got[T:2 * T])
-
-
-def workspace_16(T, k, E, H, I, has_shared):
-    """Bytes the kernels of 16-token tiles need: flags, per-token gates, tile
-    records and their columns, activations and pair outputs, token planes."""
-    def up(n):
-        return (n + 255) // 256 * 256
-
-    S = k + has_shared
-    tiles = max(min(E, T * k) + -(-T * k // 16) + (-(-T // 16) if has_shared else 0), 1)
-    return (256 + up(4 * T) + up(16 * tiles) + 256 + 2 * up(64 * tiles) + up(4 * T * S * I) + up(4 * T * S * H)
-            + 2 * up(2 * T * H) + up(T * (H // 32) * 4) + up(4 * T))
 
 
 def test_prefill_in_a_16_token_workspace(hip):
