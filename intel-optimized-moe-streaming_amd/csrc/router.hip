@@ -292,18 +292,39 @@ static void launch_select(const float* scores, int n_tokens, int n_experts, int 
 
 // Few tokens: four waves per expert row, so the n_experts x 4 waves spread
 // over the chip, and as many token accumulators as there are tokens (up to 8).
-// Above 32 tokens the number of scores decides, each step's work being
-// proportional to the hidden size on all sides (us at hidden 2048):
-//   up to 8192      the same, eight tokens at a time (64 x 16: 3.3, one wave per
-//                   expert over 16 tokens 7.2; 33 x 256: 5.7 and 7.7; 64 x 256: 7.9 and 7.7)
-//   below 49152     one wave per expert over 16 tokens, so each row is read
-//                   once per 16 tokens (128 x 256: 11.4, matrix kernel 16.8)
-//   from 49152 on   the matrix kernel (200 x 256: 16.9, vector 19.6; at hidden
-//                   1024 11.8 and 11.2, 512 x 256 12.1 and 19.8); 64 tokens a
-//                   workgroup where 32 would give well over one workgroup a CU
-//                   (2048 x 256 at hidden 1024: 20.8, 32 tokens 26.9; 1024 x
-//                   256: 17.2 and 14.7)
-constexpr int64_t RS_FEW_SCORES = 8192, RM_MIN_SCORES = 49152;
+// Above 32 tokens (us, the two kernels in turn):
+//   up to 8192 scores the same, eight tokens at a time, against one wave per
+//     expert over 16 tokens, which reads each row once per 16 tokens (4096 with
+//     fewer than 16 experts of hidden 1025 to 4096).  Hidden 2048: 64 x 16 3.3/7.2, 33
+//     x 256 5.7/7.7, 64 x 256 7.9/7.7; hidden 1536, 4096 x 2 13.1/10.1
+//   then that kernel, while its workgroups (4 experts x 16 tokens) are few enough
+//     for the chip to hold at once, four a CU, and with so few experts that most
+//     columns of a matrix tile are empty: fewer than 8, or than 12 below hidden
+//     1536.  Against the matrix kernel: 192 x 256 at hidden 1024 13.1/15.6, 2048
+//     19.8/20.7, 7168 52.7/68.3; 24576 x 2 at hidden 768 21/36; 8192 x 8 at hidden
+//     2048 27.8/22.3, 12288 x 8 at 768 20.1/23.8, 8000 x 12 at 768 22.8/17.6
+//   the matrix kernel from there on: 260 x 256 at hidden 512 13.4/12.2, 1024
+//     18.0/16.7, 2048 27.2/20.8; 128 x 512 and hidden 1024 or less 92-105 % of the
+//     other's time, and at fewer than 96 tokens (of more than 700 experts) up to
+//     107 %.  The vector kernel's fourth workgroup a CU already costs a round: there
+//     the matrix kernel is ahead from hidden 1536 on (256 x 256 at 1536 0.87, at
+//     2048 0.87) but for its long chains and idle XCDs with few tokens (768 or 1024
+//     experts 1.01-1.08, hidden 7168 up to 1.05), and with one tile of experts
+//     (4000 x 16 0.64-0.96 at every hidden size; up to 24 experts from hidden 1536
+//     on already with the third, 3072 x 16 at 2048 23.1/19.7)
+// The matrix kernel takes 64 tokens a workgroup where 32 would give well over one
+// workgroup a CU (2048 x 256 at hidden 1024: 20.8, 32 tokens 26.9; 1024 x 256:
+// 17.2 and 14.7), except under 16 experts (16384 x 8 at hidden 1536: 44.6 and 32.4).
+static int64_t route_few_scores(int hidden, int n_experts) {
+    return n_experts < 16 && hidden > 1024 && hidden <= 4096 ? 4096 : 8192;
+}
+static bool route_on_matrix(int n_tokens, int hidden, int n_experts) {
+    if (hidden < 512 || n_experts < (hidden >= 1536 ? 8 : 12)) return false;
+    const int64_t wg = (int64_t)((n_experts + 3) / 4) * ((n_tokens + 15) / 16);   // the vector kernel's
+    if (wg > 4 * 256) return hidden >= 1536 || n_tokens >= 96;
+    if (n_experts <= 24 && hidden >= 1536) return wg >= 3 * 256;
+    return wg > 3 * 256 && (n_experts <= 32 || (hidden >= 1536 && n_experts <= (hidden <= 4096 ? 512 : 128)));
+}
 constexpr int64_t RM_WIDE_TILES = 384;
 hipError_t launch_route_scores(const float* x, int n_tokens, int hidden, const float* w, int n_experts, float* scores,
                                hipStream_t stream) {
@@ -311,9 +332,11 @@ hipError_t launch_route_scores(const float* x, int n_tokens, int hidden, const f
     if (n_tokens == 1) launch_scores<4, 1>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else if (n_tokens == 2) launch_scores<4, 2>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else if (n_tokens <= 4) launch_scores<4, 4>(x, n_tokens, hidden, w, n_experts, scores, stream);
-    else if (n_tokens <= 32 || n <= RS_FEW_SCORES) launch_scores<4, 8>(x, n_tokens, hidden, w, n_experts, scores, stream);
-    else if (n < RM_MIN_SCORES || hidden < 512) launch_scores<1, 16>(x, n_tokens, hidden, w, n_experts, scores, stream);
-    else if (hidden >= 1024 && (int64_t)((n_tokens + 31) / 32) * ((n_experts + 31) / 32) > RM_WIDE_TILES)
+    else if (n_tokens <= 32 || n <= route_few_scores(hidden, n_experts))
+        launch_scores<4, 8>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else if (!route_on_matrix(n_tokens, hidden, n_experts)) launch_scores<1, 16>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else if (hidden >= 1024 && n_experts >= 16 &&
+             (int64_t)((n_tokens + 31) / 32) * ((n_experts + 31) / 32) > RM_WIDE_TILES)
         launch_scores_mfma<2>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else launch_scores_mfma<1>(x, n_tokens, hidden, w, n_experts, scores, stream);
     return hipGetLastError();

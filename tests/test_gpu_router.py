@@ -251,8 +251,9 @@ def test_routed_decode_matches_the_oracle_layer(oracle_mod, E, types, sh_types, 
 
 
 @pytest.mark.parametrize("T,H,E,k", [
-    (192, 512, 256, 8),     # the first size on the matrix kernel: whole tiles, half the waves idle
-    (1025, 516, 49, 4),     # one token and 17 experts past a tile, four columns past a pass
+    (257, 512, 256, 8),     # one token past a tile, one pass a wave
+    (1409, 516, 49, 4),     # one token and 17 experts past a tile, four columns past a pass
+    (3153, 768, 16, 2),     # half a tile of experts
     (257, 1540, 193, 6),    # the longer chains, every edge ragged
     (2048, 1024, 256, 8),   # 64 tokens a workgroup, chains of 8
     (1633, 2044, 250, 8),   # 64 tokens a workgroup, chains of 16, every edge ragged
@@ -309,3 +310,30 @@ def test_routed_scores_in_and_out_of_the_workspace():
         torch.cuda.synchronize()
         for a, b, c in zip((want, ids, weights), first, got):
             assert torch.equal(a, b) and torch.equal(a, c)
+
+
+@pytest.mark.parametrize("T,H,E,part,matrix", [
+    (25000, 768, 2, 6000, False),     # few experts: a matrix tile's columns are empty
+    (6200, 1024, 8, 1500, False),
+    (6200, 1536, 8, 1500, True),
+    (192, 1024, 256, 64, False),      # three vector workgroups a CU
+    (256, 7168, 192, 64, False),
+    (48, 1024, 1024, 33, False),
+    (256, 1024, 256, 64, False),      # four, below hidden 1536
+    (256, 1536, 256, 64, True),
+    (260, 1024, 256, 64, True),       # more than four
+    (80, 1024, 1024, 33, False),      # too few tokens
+    (3153, 512, 16, 1024, True),      # one tile of experts
+    (4096, 1536, 2, 8192, False),     # few scores: sixteen tokens a wave, as for twice as many
+])
+def test_route_scores_kernel_of_a_size(T, H, E, part, matrix):
+    """Which kernel makes a prompt's scores, by their bits: the vector kernel's are
+    the same in a part of the prompt (or a longer one) that is certainly on it;
+    the matrix kernel adds in another order."""
+    rng = np.random.default_rng(T + E)
+    x = rng.standard_normal((max(T, part), H)).astype(np.float32)
+    w = (rng.standard_normal((H, E)) * 0.05).astype(np.float32)
+    n = min(T, part)
+    whole = gpu_route(x[:T], w, 1, with_scores=True)[2]
+    vector = gpu_route(x[:part], w, 1, with_scores=True)[2]
+    assert np.array_equal(whole[:n], vector[:n]) == (not matrix)
