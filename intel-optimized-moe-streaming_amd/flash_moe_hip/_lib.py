@@ -173,3 +173,16 @@ def load(path: str | os.PathLike | None = None) -> C.CDLL:
 def check(status: int, what: str) -> None:
     if status != 0:
         raise RuntimeError(f"{what} failed with status {status} ({STATUS_TEXT.get(status, 'unknown')})")
+
+
+def current_stream(device) -> int:
+    """The handle of the CUDA device's current stream, by torch's own accessor: it
+    makes no stream object (a decode call is short beside one).  Like the public
+    call it refuses other devices; asked for their index -1 the accessor would
+    answer for the current CUDA device, and a kernel would run on host pointers."""
+    import torch
+
+    if device.type != "cuda":
+        raise ValueError(f"expected a CUDA device, got {device}")
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

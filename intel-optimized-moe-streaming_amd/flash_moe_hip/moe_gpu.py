@@ -123,12 +123,7 @@ class MoeRunner:
 
     def _stream(self, stream) -> int:
         """The handle of `stream`, or of the device's current stream."""
-        import torch
-
-        if stream is not None:
-            return stream.cuda_stream
-        index = self.device.index
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+        return stream.cuda_stream if stream is not None else _lib.current_stream(self.device)
 
     def _workspace(self, n_tokens: int, top_k: int, inter: int, sh_inter: int, stream: int, extra: int = 0):
         """The workspace of a decode call and the address of `extra` bytes after

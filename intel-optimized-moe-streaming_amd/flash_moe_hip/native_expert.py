@@ -123,9 +123,7 @@ class DeltaState:
         state = self.state
         if out is None:
             out = torch.empty((nv, dv), dtype=f32, device=state.device)
-        # (the current stream's handle without a stream object: a step is shorter
-        # than this wrapper)
-        handle = stream.cuda_stream if stream is not None else torch._C._cuda_getCurrentRawStream(state.get_device())
+        handle = stream.cuda_stream if stream is not None else _lib.current_stream(state.device)
         rc = self.lib.mqh_delta_heads(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
                                       gate.data_ptr(), out.data_ptr(), nv, dk, dv, self._flags.data_ptr(), handle)
         _lib.check(rc, "mqh_delta_heads")

@@ -232,3 +232,20 @@ def test_prefill_workspace_past_the_wide_tiles(lib):
     need = [lib.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, sh) for T in (last, last + 1, 2 * last)]
     assert need[1] == need[0] > workspace_16(last + 1, k, E, H, I, sh)
     assert need[2] == workspace_16(2 * last, k, E, H, I, sh)
+
+
+def test_cpu_devices_are_refused():
+    """Decode and DeltaNet calls on a CPU device raise before any launch."""
+    import torch
+    from flash_moe_hip.moe_gpu import MoeRunner
+    from flash_moe_hip.native_expert import DeltaState
+
+    state = DeltaState(2, 4, 4, device="cpu")
+    q, v, b = torch.zeros(2, 4), torch.zeros(2, 4), torch.zeros(2)
+    with pytest.raises(ValueError):
+        state.step(q, q, v, b, b)
+    runner = MoeRunner(device="cpu")
+    with pytest.raises(ValueError):
+        runner.decode(None, None, None, None)
+    with pytest.raises(ValueError):
+        runner.decode_routed(None, None, 1)
