@@ -185,4 +185,7 @@ def current_stream(device) -> int:
     if device.type != "cuda":
         raise ValueError(f"expected a CUDA device, got {device}")
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:   # (not a public name)
+        return torch.cuda.current_stream(device).cuda_stream
+    return raw(torch.cuda.current_device() if index is None else index)

@@ -249,3 +249,19 @@ def test_cpu_devices_are_refused():
         runner.decode(None, None, None, None)
     with pytest.raises(ValueError):
         runner.decode_routed(None, None, 1)
+
+
+def test_current_stream_without_the_private_accessor(monkeypatch):
+    """The current stream's handle comes from torch's private accessor where there
+    is one, else from the public call."""
+    from types import SimpleNamespace
+
+    import torch
+    from flash_moe_hip import _lib
+
+    device = torch.device("cuda", 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=100 + d.index))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 200 + i, raising=False)
+    assert _lib.current_stream(device) == 203
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert _lib.current_stream(device) == 103
