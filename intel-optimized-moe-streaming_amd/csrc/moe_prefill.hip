@@ -486,14 +486,16 @@ constexpr int PF_STAGE_TOKENS = 4;
 
 // Workgroup 0 routes; workgroup b > 0 stages tokens 4 (b - 1) .. 4 b - 1 into
 // the token planes, one wave a token, and sets the shared expert's gate per
-// token (sigmoid(x . g_inp), shared_expert.py:221-251).
-template <int NBH, bool XBF16>
+// token (sigmoid(x . g_inp), shared_expert.py:221-251).  W is the tile width, a
+// constant: read from the arguments the pass took 0.3 us longer at 300 and 509
+// tokens (6.2 and 8.3 us).
+template <int NBH, bool XBF16, int W>
 __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParams p) {
     __shared__ int cnt[PREFILL_MAX_EXPERTS], off[PREFILL_MAX_EXPERTS], fill[PREFILL_MAX_EXPERTS];
     __shared__ int toff[PREFILL_MAX_EXPERTS];
     __shared__ int wsum[16][2];
     const int T = p.n_tokens, K = p.top_k, E = p.n_experts, TK = T * K;
-    const int W = p.tile, wl = 31 - __builtin_clz(W);   // tile width
+    constexpr int wl = __builtin_ctz(W);   // W: the tile width
     const int e = threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (blockIdx.x > 0) {
         constexpr int H = NBH * 256;
@@ -964,9 +966,11 @@ static void launch_p2_t(const PrefillParams& p, hipStream_t s, const KernelEvent
 hipError_t launch_prefill(const PrefillParams& p, hipStream_t s, const KernelEvents& ev) {
     if (p.n_tokens <= 0) return hipSuccess;
     const dim3 route_grid(1 + (p.n_tokens + PF_STAGE_TOKENS - 1) / PF_STAGE_TOKENS);
-#define MQH_ROUTE(NBH)                                                                                               \
-    if (p.x_bf16) hipLaunchKernelGGL((k_prefill_route<NBH, true>), route_grid, dim3(PF_ROUTE_THREADS), 0, s, p);     \
-    else hipLaunchKernelGGL((k_prefill_route<NBH, false>), route_grid, dim3(PF_ROUTE_THREADS), 0, s, p)
+#define MQH_ROUTE_W(NBH, W)                                                                                             \
+    if (p.x_bf16) hipLaunchKernelGGL((k_prefill_route<NBH, true, W>), route_grid, dim3(PF_ROUTE_THREADS), 0, s, p);     \
+    else hipLaunchKernelGGL((k_prefill_route<NBH, false, W>), route_grid, dim3(PF_ROUTE_THREADS), 0, s, p)
+#define MQH_ROUTE(NBH)                                                                                                  \
+    if (p.tile == PREFILL_WIDE) { MQH_ROUTE_W(NBH, PREFILL_WIDE); } else { MQH_ROUTE_W(NBH, PREFILL_TILE); }
     switch (p.hidden) {
         case 256: MQH_ROUTE(1); break;
         case 512: MQH_ROUTE(2); break;
@@ -974,6 +978,7 @@ hipError_t launch_prefill(const PrefillParams& p, hipStream_t s, const KernelEve
         default: MQH_ROUTE(8); break;
     }
 #undef MQH_ROUTE
+#undef MQH_ROUTE_W
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     if (p.tile == PREFILL_WIDE) {
