@@ -175,17 +175,14 @@ def check(status: int, what: str) -> None:
         raise RuntimeError(f"{what} failed with status {status} ({STATUS_TEXT.get(status, 'unknown')})")
 
 
-def current_stream(device) -> int:
-    """The handle of the CUDA device's current stream, by torch's own accessor: it
-    makes no stream object (a decode call is short beside one).  Like the public
-    call it refuses other devices; asked for their index -1 the accessor would
-    answer for the current CUDA device, and a kernel would run on host pointers."""
+def stream_accessor():
+    """A function of a CUDA device's index (0 or more) that gives the handle of
+    its current stream: torch's own accessor, which makes no stream object (a
+    decode call is short beside one), or the public call in a torch without it.
+    The caller refuses the index of another device (`Tensor.get_device` gives
+    -1): the accessor would answer for the current device, and a kernel would run
+    on host pointers."""
     import torch
 
-    if device.type != "cuda":
-        raise ValueError(f"expected a CUDA device, got {device}")
-    index = device.index
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is None:   # (not a public name)
-        return torch.cuda.current_stream(device).cuda_stream
-    return raw(torch.cuda.current_device() if index is None else index)
+    return getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+        lambda index: torch.cuda.current_stream(index).cuda_stream)

@@ -70,6 +70,9 @@ class MoeRunner:
         import torch
 
         self.device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
+        # its index (None: the current one; -1: no CUDA device, refused by every call)
+        self._index = self.device.index if self.device.type == "cuda" else -1
+        self._stream_of = _lib.stream_accessor()
         self.lib = _lib.load()
         self._local = threading.local()
 
@@ -123,7 +126,16 @@ class MoeRunner:
 
     def _stream(self, stream) -> int:
         """The handle of `stream`, or of the device's current stream."""
-        return stream.cuda_stream if stream is not None else _lib.current_stream(self.device)
+        if stream is not None:
+            return stream.cuda_stream
+        index = self._index
+        if index is None:
+            import torch
+
+            index = torch.cuda.current_device()
+        elif index < 0:
+            raise ValueError(f"expected a CUDA device, got {self.device}")
+        return self._stream_of(index)
 
     def _workspace(self, n_tokens: int, top_k: int, inter: int, sh_inter: int, stream: int, extra: int = 0):
         """The workspace of a decode call and the address of `extra` bytes after

@@ -107,6 +107,7 @@ class DeltaState:
                 raise ValueError("DeltaNet state shape mismatch")
         self._flags = torch.zeros(64, dtype=torch.int32, device=self.state.device)
         nv, dv, dk = self.shape
+        self._stream_of = _lib.stream_accessor()
         self._in_shapes = [(nv, dk), (nv, dk), (nv, dv), (nv,), (nv,)]
 
     def reset(self):
@@ -123,7 +124,13 @@ class DeltaState:
         state = self.state
         if out is None:
             out = torch.empty((nv, dv), dtype=f32, device=state.device)
-        handle = stream.cuda_stream if stream is not None else _lib.current_stream(state.device)
+        if stream is not None:
+            handle = stream.cuda_stream
+        else:
+            index = state.get_device()
+            if index < 0:
+                raise ValueError(f"expected a CUDA device, got {state.device}")
+            handle = self._stream_of(index)
         rc = self.lib.mqh_delta_heads(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
                                       gate.data_ptr(), out.data_ptr(), nv, dk, dv, self._flags.data_ptr(), handle)
         _lib.check(rc, "mqh_delta_heads")

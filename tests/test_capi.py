@@ -259,9 +259,8 @@ def test_current_stream_without_the_private_accessor(monkeypatch):
     import torch
     from flash_moe_hip import _lib
 
-    device = torch.device("cuda", 3)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=100 + d.index))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda i: SimpleNamespace(cuda_stream=100 + i))
     monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 200 + i, raising=False)
-    assert _lib.current_stream(device) == 203
+    assert _lib.stream_accessor()(3) == 203
     monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
-    assert _lib.current_stream(device) == 103
+    assert _lib.stream_accessor()(3) == 103
