@@ -389,19 +389,6 @@ __device__ __forceinline__ void decode16(const uint8_t* blk, int t, float out[16
     }
 }
 
-// Runtime-type dispatch; `type` is uniform across the wavefront, so the
-// branch does not diverge.
-__device__ __forceinline__ void decode8_any(int type, const uint8_t* blk, int t, float out[8]) {
-    switch (type) {
-        case T_Q8_0: decode8<T_Q8_0>(blk, t, out); break;
-        case T_IQ4_NL: decode8<T_IQ4_NL>(blk, t, out); break;
-        case T_Q3_K: decode8<T_Q3_K>(blk, t, out); break;
-        case T_Q4_K: decode8<T_Q4_K>(blk, t, out); break;
-        case T_Q5_K: decode8<T_Q5_K>(blk, t, out); break;
-        default:     decode8<T_Q6_K>(blk, t, out); break;
-    }
-}
-
 // ------------------------------------------------------------ reductions
 
 // Sum over aligned groups of `width` lanes (width a power of two <= 64);

@@ -59,7 +59,7 @@ static int gen_units(int cols) {
 // pass is straight-line code: the loads of all its units of both rows are issued
 // before the first is used (one row and one unit at a time, behind a branch on
 // the type per unit, left a wave with one load in flight).  Two sums a row, by
-// the parity of the unit.
+// the parity of the unit's place in the pass (with NJ = 1 one sum holds all).
 template <int T, int NJ, bool RX, bool RW>
 __device__ __forceinline__ void gen_dot2(const uint8_t* W0, int r0, const uint8_t* W1, int r1, const float* x, int n8,
                                          int lp, int L, float& out0, float& out1) {

@@ -66,19 +66,6 @@ __device__ __forceinline__ void pf_stage_load(const void* src, int64_t row, bool
     }
 }
 
-// Hands the loaded words through an empty asm statement placed after the
-// weight prefetch: everything computed from them is then ordered after the
-// prefetch (the instruction selector is otherwise free to put the row's
-// arithmetic, and its wait for the row, ahead of the prefetch loads).
-template <int K, bool BF16>
-__device__ __forceinline__ void pf_stage_pin(PfStageRaw<K, BF16>& raw) {
-#pragma unroll
-    for (int it = 0; it < PfStageRaw<K, BF16>::NIT; ++it)
-#pragma unroll
-        for (int j = 0; j < (BF16 ? 1 : 2); ++j)
-            __asm__ volatile("" : "+v"(raw.r[it][j].x), "+v"(raw.r[it][j].y), "+v"(raw.r[it][j].z), "+v"(raw.r[it][j].w));
-}
-
 // The values of pass `it` (8 per lane) from the loaded words; zero past K
 template <int K, bool BF16>
 __device__ __forceinline__ void pf_raw_vals(const PfStageRaw<K, BF16>& raw, int it, int c, float v[8]) {

@@ -9,15 +9,16 @@
 //
 // Four launches, no inter-workgroup synchronisation:
 //   P0 k_prefill_route     workgroup 0 buckets the (token, slot) pairs by expert and
-//                          cuts each expert's tokens into tiles of 16; the others
+//                          cuts each expert's tokens into tiles of 16 or 64; the others
 //                          stage every token once as the B operand (token planes)
 //                          and the shared expert's sigmoid gate.
 //   P1 k_prefill_gate_up   (I/64) x max_tiles workgroups: 64 intermediate rows x one tile,
 //                          SwiGLU fused.
 //   P2 k_prefill_down      (H/128) x max_tiles workgroups: 128 output rows x one tile.
 //   P3 k_prefill_combine   grid (H/256, T): the weighted sum in top-k order.
-// With many tokens per expert the tiles are 64 tokens and P1/P2 are the kernels
-// of moe_prefill_wide.hip.
+// P1 and P2 here take tiles of 16 tokens.  With many tokens per expert and matrices
+// large enough the tiles are 64 tokens and P1/P2 are the kernels of
+// moe_prefill_wide.hip.
 //
 // P1/P2 are MFMA GEMMs (v_mfma_f32_16x16x32_f16, FP32 accumulate) whose weight
 // operand is built in registers straight from the quantized blocks as exact
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(PF_ROUTE_THREADS) void k_prefill_route(PrefillParam
         if (w < wave) { bc += wsum[w][0]; bt += wsum[w][1]; }
         tott += wsum[w][1];
     }
-    // the shared expert's tiles come first (tile j: tokens 16 j .. 16 j + 15):
+    // the shared expert's tiles come first (tile j: tokens W j .. W j + W - 1):
     // they are the fullest tiles and, with a shared expert of another type, the
     // slowest, so they start in the launch's first round rather than its tail
     const int nsh = p.has_shared ? (T + W - 1) >> wl : 0;

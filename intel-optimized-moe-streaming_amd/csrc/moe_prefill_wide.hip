@@ -4,8 +4,8 @@
 // and hold a tile's whole K in LDS; with 128 tokens an expert that rebuilds each
 // operand eight times (a 4096-token prompt: gate/up 564 us, down 676 us, the
 // matrix cores a tenth busy).  Here a tile is up to 64 tokens of one expert, in
-// NS = 1..4 column blocks of 16, and an operand built in registers serves all of
-// them:
+// NS = 1, 2 or 4 column blocks of 16, and an operand built in registers serves all
+// of them:
 //
 //   W1 k_prefill_gate_up_wide  128 intermediate rows x one tile a workgroup, 16
 //                              gate rows and the same 16 up rows a wave, SwiGLU
@@ -25,7 +25,7 @@
 // Bound by vector arithmetic (a stage's operands and scales take 1.5 times as
 // long as its MFMAs) that two waves a SIMD do not fully overlap with the matrix
 // cores; 4096 BF16 tokens, 256 experts, top-8 + shared, Q4_K/Q6_K: W1 564 -> 315
-// us, W3 676 -> 510 us, W2 28 us.  (Four waves a SIMD on one row block each,
+// us, W3 676 -> 510 us, W2 26 us.  (Four waves a SIMD on one row block each,
 // 128 registers, spilling: 345 and 483.)
 #include <hip/hip_ext.h>
 

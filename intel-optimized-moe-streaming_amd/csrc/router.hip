@@ -10,13 +10,14 @@
 //            multiplies by fl32(w), moe_layer.py:70,85-86); a non-finite or
 //            non-positive exponential sum gives 1/k each (router.py:161-166).
 //
-// Two launches.  k_route_scores (up to a hundred or so tokens): each workgroup owns 4/SPLIT experts and a
-// group of tokens; SPLIT waves share one expert row, each summing a contiguous
-// share of the hidden dimension with 16-byte loads (a lane's chain, then a
-// fixed DPP tree over the wave), and the shares are added in wave order, so
-// the summation order of a score is fixed for a given SPLIT.  k_route_scores_mfma
-// (more tokens): the same FP32 products and sums as a matrix product on the FP32
-// matrix instructions, also in a fixed order.
+// Two launches.  k_route_scores: each workgroup owns 4/SPLIT experts and a group
+// of tokens; SPLIT waves share one expert row, each summing a contiguous share of
+// the hidden dimension with 16-byte loads (a lane's chain, then a fixed DPP tree
+// over the wave), and the shares are added in wave order, so the summation order
+// of a score is fixed for a given SPLIT.  k_route_scores_mfma, for more scores
+// than that kernel makes in one round of the chip (route_on_matrix): the same
+// FP32 products and sums as a matrix product on the FP32 matrix instructions,
+// also in a fixed order.
 // k_route_select: one wavefront per token takes the top k by k rounds of a
 // wave maximum over (score, expert) keys (route_topk.h): NaN ranks above every
 // number, as np.argsort places NaN last (a NaN among the selected then makes
