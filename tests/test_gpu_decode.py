@@ -675,9 +675,10 @@ def test_intermediate_2048_over_slot_limit_falls_back(hip, oracle_mod):
 def test_generic_sizes(hip, oracle_mod, gt, ut, dt, H, I, sh_I, k, T):
     """The FP32 kernels over sizes that are no power of two, against float64.
 
-    A row's sum is two chains of at most 40 products a lane under six tree
-    levels: about sqrt(20 + 7) 2^-24 = 3e-7 of its terms' norm, which two sums
-    in turn and Q4_K's offsets (terms a few times the result) take to ~2e-6."""
+    A row's sum is two chains of at most 48 products a lane (nine units in three
+    passes: six in one chain) under six tree levels: about sqrt(24 + 7) 2^-24 =
+    3.3e-7 of its terms' norm, which two sums in turn and Q4_K's offsets (terms a
+    few times the result) take to ~2e-6."""
     t = {"gate": gt, "up": ut, "down": dt}
     E = 10
     # (scales at which the FP16 graph stays finite)

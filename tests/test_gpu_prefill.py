@@ -305,6 +305,9 @@ def test_prefill_q8_0_down_without_shared(oracle_mod, hip, shape):
     ((14, 13), "same", (512, 512), True),
     ((11, 14), "q6k", (512, 2048), True),
     ((13, 14), "none", (256, 256), True),
+    ((12, 12), "q6k", (1024, 256), True),    # gate, up and down of another type than the shared expert's
+    ((13, 13), "q6k", (512, 512), False),
+    ((11, 12), "same", (2048, 256), False),  # FP32 tokens of the largest hidden size
 ])
 def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     """Many tokens per expert (64-token tiles): experts of 0, 1, 16, 17, 32, 33,
@@ -312,7 +315,8 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     one column, and one super-block of hidden or intermediate up to eight.  The
     161 tokens are checked against the oracle; the prompt repeats them until its
     size is the wide tiles' (every repetition's rows are the same bits: a pair's
-    result does not depend on its column)."""
+    result does not depend on its column).  Alone they run on 16-token tiles, with
+    the same bits."""
     (gt, dt), (H, I) = types, shape
     kinds = {"gate": gt, "up": gt, "down": dt}
     st = {"none": None, "same": kinds, "q6k": {"gate": 14, "up": 14, "down": 14}}[sh]
@@ -323,7 +327,7 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     first = rng.permutation(first)
     # the repetitions' second pairs go to expert 0 and theirs, too, to 7: the
     # other experts keep the counts above
-    reps = 100 if H == 256 else 13
+    reps = 100 if H == 256 else 20 if I == 256 else 13
     X1 = rng.standard_normal((T, H)).astype(np.float32) * rng.uniform(0.01, 30, (T, 1)).astype(np.float32)
     X = np.concatenate([X1] * reps)
     ids = np.zeros((T * reps, 2), np.int64)
@@ -341,6 +345,29 @@ def test_prefill_wide_tiles(oracle_mod, hip, types, sh, shape, x_bf16):
     check(oracle_mod, layer, host, shared, X[T:T + 9], ids[T:T + 9], ws[T:T + 9], got[T:T + 9], "expert 7")
     for r in range(2, reps):
         np.testing.assert_array_equal(got[r * T:(r + 1) * T], got[T:2 * T])
+    alone, status = run_prefill(layer, X[:T], ids[:T], ws[:T], x_bf16=x_bf16)
+    assert status == 0 and hip.mqh_last_prefill_tile() == 16
+    np.testing.assert_array_equal(got[:T], alone)
+
+
+def test_prefill_wide_tiles_out_of_range_ids(hip):
+    """Ids out of range on 64-token tiles are flagged and contribute nothing: the
+    same bits as on 16-token tiles, with tokens of no, one and two such ids."""
+    t = {"gate": 12, "up": 12, "down": 14}
+    E, H, I, T, n = 8, 512, 512, 2400, 160
+    layer, _, _ = make_layer(7300, E, H, I, t, shared_types=t)
+    rng = np.random.default_rng(7300)
+    X = rng.standard_normal((T, H)).astype(np.float32)
+    ids = rng.integers(-2, E + 2, size=(T, 2)).astype(np.int32)
+    ws = rng.dirichlet(np.ones(2), size=T).astype(np.float32)
+    bad = ((ids < 0) | (ids >= E)).sum(axis=1)
+    assert all((bad[:n] == i).any() for i in range(3))
+    print("prefill wide tiles: ids out of range", flush=True)
+    got, status = run_prefill(layer, X, ids, ws)
+    assert status == -9 and hip.mqh_last_prefill_tile() == 64
+    alone, status = run_prefill(layer, X[:n], ids[:n], ws[:n])
+    assert status == -9 and hip.mqh_last_prefill_tile() == 16
+    np.testing.assert_array_equal(got[:n], alone)
 
 
 def test_prefill_in_a_16_token_workspace(hip):
@@ -423,5 +450,7 @@ def test_prefill_tile_width(hip, types, sh, shape, E, k, T, tile):
     print(f"prefill tile width {types} H={H} I={I} E={E} k={k} T={T}", flush=True)
     runner = MoeRunner()
     y = runner.prefill(layer, x, ids, w)
+    # (a new runner's workspace is what the query call says, to the byte)
+    assert runner._ws.numel() == hip.mqh_moe_prefill_workspace_bytes(T, k, E, H, I, int(sh))
     assert runner.status() == 0 and bool(torch.isfinite(y).all())
     assert hip.mqh_last_prefill_tile() == tile

@@ -261,17 +261,27 @@ def test_routed_decode_matches_the_oracle_layer(oracle_mod, E, types, sh_types, 
 def test_route_scores_many_tokens(T, H, E, k):
     """Scores against float64: an FP32 sum of H products in any order is off by at
     most H eps sum|x w| (eps = 2^-24), and each edge has inputs of its own size, so
-    a column, row or expert taken twice or left out shows."""
+    a column, row or expert taken twice or left out shows.  Over all scores,
+    chains of L products under about ten more sums are off by sqrt(L / 2 + 10) eps
+    / sqrt(3), 1.5e-7 at L = 16; operands of fewer bits would be off by 1e-4.  The
+    selection is the top k of these scores and their softmax."""
     rng = np.random.default_rng(T + H + E)
     x = rng.standard_normal((T, H)).astype(np.float32)
     w = (rng.standard_normal((H, E)) * 0.05).astype(np.float32)
     x[-1] *= 3.0
     x[:, -1] += 2.0
     w[:, -1] += 0.5
-    _, _, scores = gpu_route(x, w, k, with_scores=True)
+    ids, weights, scores = gpu_route(x, w, k, with_scores=True)
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    exact = x64 @ w64
     bound = H * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
-    assert np.all(np.abs(scores - x64 @ w64) <= bound)
+    assert np.all(np.abs(scores - exact) <= bound)
+    assert np.linalg.norm(scores - exact) <= 3e-7 * np.linalg.norm(exact)
+    want = np.argsort(-scores, axis=1, kind="stable")[:, :k]
+    np.testing.assert_array_equal(ids, want)
+    top = np.take_along_axis(scores, want, axis=1).astype(np.float64)
+    e = np.exp(top - top[:, :1])
+    np.testing.assert_allclose(weights, e / e.sum(axis=1, keepdims=True), rtol=0, atol=2e-6)
 
 
 def test_routed_scores_in_and_out_of_the_workspace():
