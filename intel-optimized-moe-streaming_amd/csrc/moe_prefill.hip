@@ -101,42 +101,42 @@ constexpr int pf_occupancy(int lds_bytes) {
 // pay for it with few, long workgroups (128 x 64 or 256 x 64 outputs, one or two
 // a CU, 256 columns a stage) and the pass that makes the activation planes, so
 // they need the more of it the smaller the matrices are.  The amount is
-// pairs sqrt(pairs per expert) hidden inter, or without the matrix size at
-// hidden 256, whose down projection has one workgroup a tile.
+// pairs cbrt(pairs per expert) hidden inter, or without the matrix size at
+// hidden 256, whose down projection has one workgroup a tile (the exponents and
+// amounts fit 8562 layers measured on both widths).
 //
 // Layer times in us, 64-token and 16-token tiles, BF16 tokens of 128 or 256
 // experts, top-8 (Q4_K/Q6_K with a shared expert, Q3_K with one in Q6_K):
 //   hidden x inter     2048x512           1024x256          512x512           512x256
 //   pairs (an expert)
 //   Q4_K/Q6_K
-//      6192   (48)   241/251 (1.1)     104/89  (.28)     102/82  (.28)      76/61  (.14)
-//     16452   (64)   495/616 (3.5)     181/199 (.86)     175/180 (.86)     123/122 (.43)
-//     32904  (128)   852/1174 (9.8)    331/376 (2.4)     312/332 (2.4)     201/218 (1.2)
+//      6192   (48)   241/251  (1.5)    104/89   (0.36)   102/82   (0.36)   76/61    (0.18)
+//     16452   (64)   495/616  (4.2)    181/199  (1.1)    175/180  (1.1)    123/122  (0.53)
+//     32904  (128)   852/1174 (11)     331/376  (2.7)    312/332  (2.7)    201/218  (1.3)
 //   Q5_K
-//      6144   (48)   213/239 (1.5)      71/85  (.37)      90/79  (.37)      67/57  (.19)
-//     16384   (64)   425/605 (4.6)     161/184 (1.1)     163/171 (1.1)     110/118 (.57)
+//      6144   (48)   213/239  (2.9)    71/85    (0.73)   90/79    (0.73)   67/57    (0.37)
+//     16384   (64)   425/605  (8.6)    161/184  (2.1)    163/171  (2.1)    110/118  (1.1)
 //   Q3_K
-//      4131   (32)   199/197 (2.0)      90/79  (.51)      81/80  (.51)      64/57  (.25)
-//      8262   (64)   249/339 (5.8)     109/128 (1.5)     104/128 (1.5)      77/86  (.72)
+//      4131   (32)   199/197  (3.1)    90/79    (0.79)   81/80    (0.79)   64/57    (0.39)
+//      8262   (64)   249/339  (7.9)    109/128  (2)      104/128  (2)      77/86    (0.99)
 //   Q6_K
-//      4096   (32)   259/276 (3.4)      91/99  (.87)      90/109 (.87)      61/71  (.43)
-//      8192   (64)   399/472 (9.9)     158/171 (2.4)     143/183 (2.4)     105/113 (1.2)
+//      4096   (32)   259/276  (6.8)    91/99    (1.7)    90/109   (1.7)    61/71    (0.85)
+//      8192   (64)   399/472  (17)     158/171  (4.3)    143/183  (4.3)    105/113  (2.1)
 // (in parentheses the amount over the type's threshold).  Hidden 256, inter 512,
 // 65536 pairs, 256 an expert: 403/349 in Q4_K, 374/338 in Q5_K, 397/441 in Q3_K,
-// 545/558 in Q6_K; 8192 pairs, 32 an expert: 96/67, 75/66, 93/81, 110/100.  Half
-// as wide a matrix needs twice the pairs (gate/up has pairs inter / 8192
-// workgroups, one a CU from there on): 4131 pairs of hidden 2048, inter 256 in
-// Q6_K with a shared expert take 22 % longer in 64-token tiles.
+// 545/558 in Q6_K; 8192 pairs, 32 an expert: 96/67, 75/66, 93/81, 110/100.  A
+// shared expert's tiles, the fullest, start first and count against the wide ones
+// (4131 pairs of hidden 2048, inter 256 in Q6_K, with one: 22 % slower).
 // Below PF_WIDE_TOKENS (hidden 2048, inter 512, 18 and 36 pairs an expert):
 // Q4_K/Q6_K 303/298 and 366/423, Q3_K 310/286 and 399/468, Q6_K 433/396 and
 // 538/601; Q5_K, 16 and 32 an expert, 275/258 and 326/405.  Below PF_WIDE_PAIRS
 // it depends on the type (256 tokens of 16 experts, 2304 pairs: 126/120 in Q3_K,
 // 93/101 in Q4_K, 88/94 in Q5_K, 133/152 in Q6_K); the line is the slowest type's.
 constexpr int64_t PF_WIDE_TOKENS = 32, PF_WIDE_PAIRS = 4096;
-static double pf_wide_work(int gate_type, int hidden) {
-    const bool q36 = gate_type == T_Q3_K || gate_type == T_Q6_K;
-    if (hidden == 256) return q36 ? 4e5 : 2e6;
-    return gate_type == T_Q6_K ? 7e9 : gate_type == T_Q3_K ? 1.2e10 : gate_type == T_Q5_K ? 3e10 : 4e10;
+static double pf_wide_work(int gate_type, int hidden, int has_shared) {
+    const int i = gate_type == T_Q4_K ? 0 : gate_type == T_Q5_K ? 1 : gate_type == T_Q3_K ? 2 : 3;
+    constexpr double at_256[4] = {5.6e5, 4.4e5, 1.2e5, 1.2e5}, above[4] = {1.3e10, 8e9, 3.5e9, 2e9};
+    return hidden == 256 ? at_256[i] : above[i] * (has_shared ? 1.25 : 1.0);
 }
 
 #ifndef PF_OCC_GU
@@ -829,11 +829,12 @@ int prefill_wide_max_tokens(int slots, int hidden, int inter) {
 bool prefill_wide_size(int n_tokens, int top_k, int n_experts, int hidden, int inter, int has_shared, int gate_type) {
     const int64_t P = (int64_t)n_tokens * (top_k + (has_shared ? 1 : 0));
     const int64_t experts = (top_k > 0 ? n_experts : 0) + (has_shared ? 1 : 0);
-    if (P < PF_WIDE_TOKENS * experts || P < PF_WIDE_PAIRS || P * inter < PF_WIDE_PAIRS * 512 ||
+    if (P < PF_WIDE_TOKENS * experts || P < PF_WIDE_PAIRS ||
         n_tokens > prefill_wide_max_tokens(top_k + (has_shared ? 1 : 0), hidden, inter))
         return false;
-    const double work = (double)P * std::sqrt((double)P / (double)experts);
-    return work * (hidden == 256 ? 1.0 : (double)hidden * inter) >= pf_wide_work(gate_type, hidden);
+    const double work = (double)P * std::cbrt((double)P / (double)experts);
+    return work * (hidden == 256 ? 1.0 : (double)hidden * inter) >=
+           pf_wide_work(gate_type, hidden, has_shared);
 }
 
 bool prefill_wide_types(int down_type, int has_shared, int sh_down_type) {

@@ -212,9 +212,10 @@ def workspace_16(T, k, E, H, I, has_shared):
 
 @pytest.mark.parametrize("k,E,H,I,sh,last", [
     (8, 256, 2048, 512, 1, 913),      # 32 pairs an expert
-    (8, 60, 512, 256, 1, 910),        # one gate/up workgroup a CU
+    (8, 60, 512, 256, 1, 503),        # pairs cbrt(pairs an expert) hidden inter
     (8, 8, 2048, 2048, 0, 511),       # 4096 pairs
-    (2, 8, 256, 2048, 0, 5428),       # pairs sqrt(pairs an expert)
+    (2, 8, 256, 2048, 0, 5421),       # pairs cbrt(pairs an expert)
+    (8, 256, 256, 256, 1, 2868),
 ])
 def test_prefill_workspace_of_prompts_below_the_wide_tiles(lib, k, E, H, I, sh, last):
     """Only prompts that some type takes 64-token tiles for pay for their planes."""

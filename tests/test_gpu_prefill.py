@@ -354,7 +354,7 @@ def test_prefill_wide_tiles_out_of_range_ids(hip):
     """Ids out of range on 64-token tiles are flagged and contribute nothing: the
     same bits as on 16-token tiles, with tokens of no, one and two such ids."""
     t = {"gate": 12, "up": 12, "down": 14}
-    E, H, I, T, n = 8, 512, 512, 2400, 160
+    E, H, I, T, n = 8, 512, 512, 2700, 160
     layer, _, _ = make_layer(7300, E, H, I, t, shared_types=t)
     rng = np.random.default_rng(7300)
     X = rng.standard_normal((T, H)).astype(np.float32)
@@ -425,11 +425,10 @@ def test_prefill_in_a_16_token_workspace(hip):
     ((13, 13), False, (512, 512), 60, 8, 1536, 64),
     ((11, 11), False, (512, 256), 60, 8, 520, 16),
     ((11, 11), False, (512, 512), 60, 8, 768, 64),
-    ((14, 14), False, (512, 256), 60, 8, 600, 16),
-    ((14, 14), False, (512, 256), 60, 8, 1024, 64),
-    # one super-block of intermediate: twice the pairs
-    ((14, 14), False, (2048, 256), 128, 8, 512, 16),
-    ((14, 14), False, (2048, 256), 128, 8, 1024, 64),
+    ((14, 14), False, (512, 256), 60, 8, 520, 64),
+    ((14, 14), True, (512, 256), 60, 8, 480, 16),     # (a shared expert asks for a quarter more)
+    ((14, 14), True, (512, 256), 60, 8, 600, 64),
+    ((14, 14), False, (2048, 256), 16, 8, 512, 64),
     ((12, 8), False, (2048, 512), 8, 2, 4096, 16),
 ])
 def test_prefill_tile_width(hip, types, sh, shape, E, k, T, tile):
