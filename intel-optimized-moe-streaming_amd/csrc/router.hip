@@ -335,7 +335,8 @@ hipError_t launch_route_scores(const float* x, int n_tokens, int hidden, const f
     else if (n_tokens <= 4) launch_scores<4, 4>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else if (n_tokens <= 32 || n <= route_few_scores(hidden, n_experts))
         launch_scores<4, 8>(x, n_tokens, hidden, w, n_experts, scores, stream);
-    else if (!route_on_matrix(n_tokens, hidden, n_experts)) launch_scores<1, 16>(x, n_tokens, hidden, w, n_experts, scores, stream);
+    else if (!route_on_matrix(n_tokens, hidden, n_experts))
+        launch_scores<1, 16>(x, n_tokens, hidden, w, n_experts, scores, stream);
     else if (hidden >= 1024 && n_experts >= 16 &&
              (int64_t)((n_tokens + 31) / 32) * ((n_experts + 31) / 32) > RM_WIDE_TILES)
         launch_scores_mfma<2>(x, n_tokens, hidden, w, n_experts, scores, stream);
